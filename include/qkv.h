@@ -136,6 +136,13 @@ int qkv_int4_pack_k(const void* key, const int64_t* k_strides, int64_t batch, in
 int qkv_int4_select_channels(const uint8_t* packed, const uint16_t* scales, int64_t rows,
                              int64_t tokens, int64_t capacity, int64_t head_dim, int64_t group,
                              int64_t selected, uint64_t* stats, int32_t* chan_idx, void* stream);
+/* The same with caller-owned scratch for the chunks' partial sums (8-byte
+ * aligned, contents irrelevant): two launches and no atomics. */
+int64_t qkv_int4_select_channels_workspace_bytes(int64_t rows, int64_t tokens, int64_t head_dim);
+int qkv_int4_select_channels_ws(const uint8_t* packed, const uint16_t* scales, int64_t rows,
+                                int64_t tokens, int64_t capacity, int64_t head_dim, int64_t group,
+                                int64_t selected, uint64_t* stats, int32_t* chan_idx,
+                                void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Subset slab of tokens [t_begin, t_end): the `selected` channels chan_idx
  * of each K row re-quantized as one int4 group.  slab holds rows *

@@ -42,6 +42,8 @@ _PROTOTYPES = {
                                    _f32, _vp]),
     "qkv_int4_pack_k": (_i32, [_vp, _P(_i64), _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _i64, _i32, _vp]),
     "qkv_int4_select_channels": (_i32, [_vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp]),
+    "qkv_int4_select_channels_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "qkv_int4_select_channels_ws": (_i32, [_vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp]),
     "qkv_int4_build_slab": (_i32, [_vp, _P(_i64), _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp,
                                    _i64, _i32, _vp]),
     "qkv_int4_query_words": (_i32, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _i32, _vp]),

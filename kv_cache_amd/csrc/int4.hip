@@ -43,123 +43,227 @@ __device__ __forceinline__ void halfx8(const uint4& raw, float* x) {
   x[6] = half_lo<F16>(raw.w); x[7] = half_hi<F16>(raw.w);
 }
 
-// Quantizes 8 values against the group amax `a` (already reduced) and packs
-// them into one little-endian word of nibbles (channel i at bits 4i..4i+3).
-__device__ __forceinline__ uint32_t quantize8(const float* x, float a, uint32_t* sbits_out) {
-  uint32_t sbits = f32_to_f16bits_sat(a / 7.0f);
-  float s = f16bits_to_f32(sbits);
-  uint32_t word = 0;
-  if (s != 0.0f) {
+// The fp16 scale of a group with amax `a` >= 0: fp16(fp32(a / 7)), saturated.
+// a holds at most 11 significant bits, so a / 7 is either exactly an fp16
+// rounding boundary or at least 2^-15 (relative) away from every one: one
+// Newton step on a * fp32(1/7) (exact where the quotient is representable)
+// rounds to the same fp16 as the IEEE division, in 3 instructions.
+__device__ __forceinline__ uint32_t group_scale(float a) {
+  a = fminf(a, 3.4028235e38f);   // (an infinite amax saturates as it did)
+  const float r7 = 1.0f / 7.0f;
+  const float q = a * r7;
+  return f32_to_f16bits_sat(__builtin_fmaf(__builtin_fmaf(-7.0f, q, a), r7, q));
+}
+
+// Reciprocal of a scale for codes8, 0 for the all-zero group's scale 0.
+__device__ __forceinline__ float code_rcp(float s) { return s != 0.0f ? __builtin_amdgcn_rcpf(s) : 0.0f; }
+
+// Eight codes clamp(rint_even(x / s), -8, 7) as one little-endian word of
+// nibbles (channel i at bits 4i..4i+3), rs ~ 1/s.  x and s have at most 11
+// significant bits, so x / s is either exactly half-way between two integers
+// or at least 2^-13.1 away from every such point (below 128 in magnitude).
+// fma(x, rs, 384) rounds the quotient to multiples of 2^-15: an approximate
+// quotient of a tie lands exactly on it, any other stays on its side.  Adding
+// 1.5 * 2^23 - 384 rounds to the nearest integer, ties to even, leaving
+// 0x4B400000 + code in the bits; the codes are gathered by shift-and-add
+// (the constants' sum is known) as (code + 8) nibbles, then xor 8.  4.3
+// instructions a value; the IEEE division with rint, conversion and masking
+// took about 20 and bound the pack kernel.
+__device__ __forceinline__ uint32_t codes8(const float* x, float rs) {
+  uint32_t acc = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) word |= (static_cast<uint32_t>(int4_code(x[i], s)) & 0xFu) << (4 * i);
+  for (int i = 7; i >= 0; --i) {
+    const float t = __builtin_fmaf(x[i], rs, 384.0f) + (12582912.0f - 384.0f);
+    const float c = __builtin_amdgcn_fmed3f(t, 12582904.0f, 12582919.0f);
+    acc = (acc << 4) + __float_as_uint(c);
   }
-  *sbits_out = sbits;
-  return word;
+  constexpr uint32_t kBias = 0x4B400000u + (0x4B400000u << 4) + (0x4B400000u << 8);   // higher terms vanish mod 2^32
+  return (acc - kBias + 0x88888888u) ^ 0x88888888u;
+}
+
+// Max over the LANES (4, 8 or 16) lanes of an aligned group, on the bit
+// patterns of non-negative floats.
+template <int LANES>
+__device__ __forceinline__ float group_max(float x) {
+  static_assert(LANES == 2 || LANES == 4 || LANES == 8 || LANES == 16, "lanes of a DPP row");
+  uint32_t v = __float_as_uint(x);
+  v = max(v, dpp_mov<0xB1>(v, v));
+  if constexpr (LANES >= 4) v = max(v, dpp_mov<0x4E>(v, v));
+  if constexpr (LANES >= 8) v = max(v, dpp_mov<0x141>(v, v));
+  if constexpr (LANES >= 16) v = max(v, dpp_mov<0x140>(v, v));
+  return __uint_as_float(v);
 }
 
 // ---------------------------------------------------------------------------
 // Pack: one thread per 8 channels of a token; GROUP/8 lanes share a scale.
+// A workgroup takes kPackIter * 256 * 8 / D tokens of one row, every thread's
+// kPackIter 16-byte loads issued before the first is used.
 // ---------------------------------------------------------------------------
+constexpr int kPackIter = 4;
+
 template <int GROUP, bool F16>
 __global__ __launch_bounds__(kThreads) void pack_kernel(
     const uint16_t* __restrict__ key, int64_t ksb, int64_t ksh, int64_t kst, int kv_heads,
-    int t_begin, int ntok, int head_dim, uint8_t* __restrict__ packed,
-    uint16_t* __restrict__ scales, int64_t capacity, int64_t total) {
+    int t_begin, int t_end, int tpt_log2, unsigned tiles, uint8_t* __restrict__ packed,
+    uint16_t* __restrict__ scales, int64_t capacity) {
   constexpr int TPG = GROUP / 8;
-  const int tpt = head_dim / 8;
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  const bool active = gid < total;
-  const int64_t g = active ? gid : 0;
-  const int64_t tok_lin = g / tpt;
-  const int c8 = static_cast<int>(g - tok_lin * tpt);
-  const int64_t r = tok_lin / ntok;
-  const int t = t_begin + static_cast<int>(tok_lin - r * ntok);
-  const int b = static_cast<int>(r / kv_heads), h = static_cast<int>(r % kv_heads);
-  uint4 raw = make_uint4(0, 0, 0, 0);
-  if (active) raw = *reinterpret_cast<const uint4*>(key + b * ksb + h * ksh + t * kst + c8 * 8);
-  float x[8];
-  halfx8<F16>(raw, x);
-  float a = 0.0f;
+  const unsigned r = blockIdx.x / tiles, tile = blockIdx.x - r * tiles;
+  const int b = static_cast<int>(r / static_cast<unsigned>(kv_heads));
+  const int h = static_cast<int>(r) - b * kv_heads;
+  const int c8 = threadIdx.x & ((1 << tpt_log2) - 1);
+  const int step = kThreads >> tpt_log2;   // tokens per load of the workgroup
+  const int t0 = t_begin + static_cast<int>(tile) * kPackIter * step + static_cast<int>(threadIdx.x >> tpt_log2);
+  const uint16_t* row = key + b * ksb + h * ksh + c8 * 8;
+  uint4 raw[kPackIter];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) a = fmaxf(a, fabsf(x[i]));
+  for (int it = 0; it < kPackIter; ++it) {
+    raw[it] = make_uint4(0, 0, 0, 0);
+    if (t0 + it * step < t_end)
+      raw[it] = *reinterpret_cast<const uint4*>(row + static_cast<int64_t>(t0 + it * step) * kst);
+  }
 #pragma unroll
-  for (int m = 1; m < TPG; m <<= 1) a = fmaxf(a, shfl_xor(a, m));
-  uint32_t sbits;
-  uint32_t word = quantize8(x, a, &sbits);
-  if (active) {
-    const int64_t tok = r * capacity + t;
-    reinterpret_cast<uint32_t*>(packed)[tok * tpt + c8] = word;
-    if (c8 % TPG == 0) scales[tok * (head_dim / GROUP) + c8 / TPG] = static_cast<uint16_t>(sbits);
+  for (int it = 0; it < kPackIter; ++it) {
+    const int t = t0 + it * step;
+    float x[8];
+    halfx8<F16>(raw[it], x);
+    float a = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a = fmaxf(a, fabsf(x[i]));
+    const uint32_t sbits = group_scale(group_max<TPG>(a));
+    const uint32_t word = codes8(x, code_rcp(f16bits_to_f32(sbits)));
+    if (t < t_end) {
+      const int64_t tok = static_cast<int64_t>(r) * capacity + t;
+      reinterpret_cast<uint32_t*>(packed)[(tok << tpt_log2) + c8] = word;
+      if (c8 % TPG == 0) scales[((tok << tpt_log2) + c8) / TPG] = static_cast<uint16_t>(sbits);
+    }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Channel statistic: sum_t |code| * F(scale), exact in uint64 (atomics are
-// order-free on integers, so the result is deterministic).
+// Channel statistic: sum_t |code| * F(scale), exact in uint64 (order-free).
+// A workgroup sums one chunk of a row's tokens: a thread takes 16 channels of
+// a token (8 bytes), four tokens' loads in flight; the threads' sums meet in
+// LDS.  With `part` the chunk's sums are stored there (no atomics, no zeroed
+// memory) for select_channels_kernel to add up; else they are added to
+// `stats` by atomics (integers, so the result does not depend on the order).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kThreads) void zero_u64_kernel(uint64_t* p, int64_t n) {
   int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   if (i < n) p[i] = 0;
 }
 
+// |code| of eight nibbles at once (8 for code -8).
+__device__ __forceinline__ uint32_t nibble_abs(uint32_t w) {
+  const uint32_t s = w & 0x88888888u, one = s >> 3;
+  return (w ^ (s | (s - one))) + one;
+}
+
 __global__ __launch_bounds__(kThreads) void channel_stats_kernel(
     const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scales, int tokens,
-    int64_t capacity, int head_dim, int group, int chunk, uint64_t* __restrict__ stats) {
-  __shared__ uint64_t part[kThreads * 8];
+    int64_t capacity, int head_dim, int group, int chunk, uint64_t* __restrict__ part,
+    uint64_t* __restrict__ stats) {
+  constexpr int kPad = kThreads + 8;   // channels k and k + 1 of a slot 16 banks apart
+  __shared__ uint64_t sums[16 * kPad];
   const int r = blockIdx.y;
-  const int tpt = head_dim / 8;          // threads per token
-  const int rows_per_iter = kThreads / tpt;
-  const int c8 = threadIdx.x % tpt, tl = threadIdx.x / tpt;
+  const int lpt = head_dim / 16;         // threads per token
+  const int step = kThreads / lpt;       // tokens per load of the workgroup
+  const int slot = threadIdx.x % lpt, tl = threadIdx.x / lpt;
   const int t0 = blockIdx.x * chunk, t1 = min(tokens, t0 + chunk);
   const int spt = head_dim / group;
-  uint64_t acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  const uint32_t* words = reinterpret_cast<const uint32_t*>(packed);
-  for (int t = t0 + tl; t < t1; t += rows_per_iter) {
-    const int64_t tok = static_cast<int64_t>(r) * capacity + t;
-    uint32_t w = words[tok * tpt + c8];
-    uint64_t f = fp16_fixed24(scales[tok * spt + (c8 * 8) / group]);
+  const uint2* words = reinterpret_cast<const uint2*>(packed) + static_cast<int64_t>(r) * capacity * lpt + slot;
+  const uint16_t* sc = scales + static_cast<int64_t>(r) * capacity * spt + (slot * 16) / group;
+  uint64_t acc[16] = {};
+  constexpr int U = 4;
+  for (int t = t0 + tl; t < t1; t += U * step) {
+    uint2 w[U];
+    uint32_t sb[U];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      int c = static_cast<int>(w << (28 - 4 * i)) >> 28;   // sign-extend nibble i
-      acc[i] += f * static_cast<uint64_t>(c < 0 ? -c : c);
+    for (int u = 0; u < U; ++u) {   // tokens past the chunk: scale 0 adds nothing
+      const int64_t tu = min(t + u * step, t1 - 1);
+      w[u] = words[tu * lpt];
+      sb[u] = sc[tu * spt];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint64_t f = t + u * step < t1 ? fp16_fixed24(sb[u]) : 0;
+      const uint32_t flo = static_cast<uint32_t>(f), fhi = static_cast<uint32_t>(f >> 32);
+      const uint32_t a[2] = {nibble_abs(w[u].x), nibble_abs(w[u].y)};
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] += static_cast<uint64_t>(flo) * ((a[i >> 3] >> (4 * (i & 7))) & 0xFu);
+      if (__any(fhi)) {   // scales of 256 and more
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          acc[i] += static_cast<uint64_t>(fhi * ((a[i >> 3] >> (4 * (i & 7))) & 0xFu)) << 32;
+      }
     }
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) part[tl * head_dim + c8 * 8 + i] = acc[i];
+  for (int i = 0; i < 16; ++i) sums[i * kPad + threadIdx.x] = acc[i];
   __syncthreads();
-  for (int c = threadIdx.x; c < head_dim; c += kThreads) {
+  if (static_cast<int>(threadIdx.x) < head_dim) {
+    const int cs = threadIdx.x % lpt, ck = threadIdx.x / lpt;   // channel 16 * cs + ck
     uint64_t s = 0;
-    for (int row = 0; row < rows_per_iter; ++row) s += part[row * head_dim + c];
-    if (s) atomicAdd(reinterpret_cast<unsigned long long*>(stats + static_cast<int64_t>(r) * head_dim + c),
-                     static_cast<unsigned long long>(s));
+#pragma unroll 8
+    for (int j = 0; j < step; ++j) s += sums[ck * kPad + cs + lpt * j];
+    const int c = cs * 16 + ck;
+    if (part)
+      part[(static_cast<int64_t>(r) * gridDim.x + blockIdx.x) * head_dim + c] = s;
+    else if (s)
+      atomicAdd(reinterpret_cast<unsigned long long*>(stats + static_cast<int64_t>(r) * head_dim + c),
+                static_cast<unsigned long long>(s));
   }
 }
 
-// One wave per row: rank(c) = #{e : st[e] > st[c] or (st[e] == st[c] and e < c)};
-// the channels of rank < S are written in ascending channel order.
-__global__ __launch_bounds__(64) void select_channels_kernel(const uint64_t* __restrict__ stats,
-                                                             int head_dim, int selected,
-                                                             int32_t* __restrict__ chan_idx) {
+// One workgroup of 1024 threads per row: the statistic summed from the row's
+// `n_part` partial sums (written to `stats`), or read from `stats` (n_part =
+// 0); rank(c) = #{e : st[e] > st[c] or (st[e] == st[c] and e < c)}; the
+// channels of rank < S are written in ascending channel order.  1024 / D
+// threads share a channel's sums and its rank's compares.
+__global__ __launch_bounds__(1024) void select_channels_kernel(const uint64_t* __restrict__ part, int n_part,
+                                                               uint64_t* __restrict__ stats, int head_dim,
+                                                               int selected, int32_t* __restrict__ chan_idx) {
+  __shared__ uint64_t psum[1024];
   __shared__ uint64_t st[256];
-  const int r = blockIdx.x, lane = threadIdx.x;
-  for (int c = lane; c < head_dim; c += 64) st[c] = stats[static_cast<int64_t>(r) * head_dim + c];
+  __shared__ int rank_s[256];
+  __shared__ int wcnt[4];
+  const int r = blockIdx.x, tid = threadIdx.x;
+  const int c = tid & (head_dim - 1), q = tid / head_dim, nq = 1024 / head_dim;
+  uint64_t v = 0;
+  if (n_part) {
+    const uint64_t* p = part + static_cast<int64_t>(r) * n_part * head_dim + c;
+#pragma unroll 4
+    for (int i = q; i < n_part; i += nq) v += p[static_cast<int64_t>(i) * head_dim];
+  } else if (q == 0) {
+    v = stats[static_cast<int64_t>(r) * head_dim + c];
+  }
+  psum[tid] = v;
+  if (tid < 256) rank_s[tid] = 0;
   __syncthreads();
-  int base = 0;
-  for (int c0 = 0; c0 < head_dim; c0 += 64) {
-    const int c = c0 + lane;
-    bool sel = false;
-    if (c < head_dim) {
-      const uint64_t v = st[c];
-      int rank = 0;
-      for (int e = 0; e < head_dim; ++e) rank += (st[e] > v) || (st[e] == v && e < c);
-      sel = rank < selected;
-    }
-    const uint64_t mask = __ballot(sel);
-    if (sel) {
-      int pos = base + __popcll(mask & ((1ull << lane) - 1ull));
-      chan_idx[static_cast<int64_t>(r) * selected + pos] = c;
-    }
-    base += __popcll(mask);
+  if (tid < head_dim) {
+    uint64_t t = 0;
+    for (int j = 0; j < nq; ++j) t += psum[j * head_dim + tid];
+    st[tid] = t;
+    if (n_part) stats[static_cast<int64_t>(r) * head_dim + tid] = t;
+  }
+  __syncthreads();
+  const uint64_t own = st[c];
+  int rank = 0;
+  const int per = head_dim / nq;   // compares of this thread: 4 (D = 64), 16 or 64
+#pragma unroll 4
+  for (int i = 0; i < per; ++i) {
+    const int e = q * per + i;
+    rank += (st[e] > own) || (st[e] == own && e < c);
+  }
+  if (rank) atomicAdd(&rank_s[c], rank);
+  __syncthreads();
+  const bool sel = tid < head_dim && rank_s[c] < selected;
+  const uint64_t mask = __ballot(sel);
+  if (tid < head_dim && (tid & 63) == 0) wcnt[tid >> 6] = __popcll(mask);
+  __syncthreads();
+  if (sel) {
+    int pos = __popcll(mask & ((1ull << (tid & 63)) - 1ull));
+    for (int w = 0; w < (tid >> 6); ++w) pos += wcnt[w];
+    chan_idx[static_cast<int64_t>(r) * selected + pos] = c;
   }
 }
 
@@ -184,6 +288,73 @@ __device__ __forceinline__ int64_t slab_offset(int64_t t, int x) {
   const int b = (k - lane * KPLN) * (S / 2) + x;
   return tile * 4096 + (64 * (b >> 4) + lane) * 16 + (b & 15);
 }
+// Rows of K 16-byte aligned: one wave takes 64 tokens of a row.  The tokens'
+// whole rows are loaded with 16-byte loads, all in flight (every 128-byte
+// line of K holds selected channels, so nothing is read in vain), and staged
+// in LDS; then lane l owns token l, reads its S channels from LDS (the
+// channel ids are wave-uniform) and writes its S/2 bytes in 16-byte pieces,
+// so the scale and the codes need no other lane.  LDS rows are 16 bytes
+// longer than K's: a read's 64 lanes fall on 16 banks, 4 lanes each.
+template <int S, int D, bool F16>
+__global__ __launch_bounds__(64) void build_slab_rows_kernel(
+    const uint16_t* __restrict__ key, int64_t ksb, int64_t ksh, int64_t kst, int kv_heads,
+    int t_begin, int t_end, unsigned tiles, const int32_t* __restrict__ chan_idx,
+    uint8_t* __restrict__ slab, uint16_t* __restrict__ slab_scales, int64_t capacity) {
+  constexpr int kLds = D / 8 + 1;            // 16-byte pieces of an LDS row
+  constexpr int kTok = 512 / D;              // tokens per load of the wave
+  constexpr int kLoads = 64 / kTok;
+  constexpr int kBatch = kLoads < 16 ? kLoads : 16;
+  __shared__ uint4 rows[64 * kLds];
+  const unsigned r = blockIdx.x / tiles, tile = blockIdx.x - r * tiles;
+  const int b = static_cast<int>(r / static_cast<unsigned>(kv_heads));
+  const int h = static_cast<int>(r) - b * kv_heads;
+  const int lane = threadIdx.x;
+  const int t0 = t_begin + static_cast<int>(tile) * 64;
+  const int piece = lane % (D / 8), tl = lane / (D / 8);
+  const uint16_t* base = key + b * ksb + h * ksh + piece * 8;
+#pragma unroll
+  for (int i0 = 0; i0 < kLoads; i0 += kBatch) {
+    uint4 raw[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int k = (i0 + i) * kTok + tl;
+      raw[i] = make_uint4(0, 0, 0, 0);
+      if (t0 + k < t_end) raw[i] = *reinterpret_cast<const uint4*>(base + static_cast<int64_t>(t0 + k) * kst);
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) rows[((i0 + i) * kTok + tl) * kLds + piece] = raw[i];
+  }
+  __syncthreads();
+  const int t = t0 + lane;
+  const uint16_t* own = reinterpret_cast<const uint16_t*>(rows + lane * kLds);
+  const int32_t* idx = chan_idx + static_cast<int64_t>(r) * S;
+  float x[S];
+  float a = 0.0f;
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    // channel ids come from qkv_int4_select_channels; clamping keeps a bad id in the row
+    x[i] = half_to_f32<F16>(own[min(max(idx[i], 0), D - 1)]);
+    a = fmaxf(a, fabsf(x[i]));
+  }
+  const uint32_t sbits = group_scale(a);
+  const float rs = code_rcp(f16bits_to_f32(sbits));
+  uint32_t w[S / 8];
+#pragma unroll
+  for (int j = 0; j < S / 8; ++j) w[j] = codes8(x + 8 * j, rs);
+  if (t >= t_end) return;
+  uint8_t* out = slab + static_cast<int64_t>(r) * capacity * (S / 2);
+  if constexpr (S == 16) {
+    *reinterpret_cast<uint2*>(out + slab_offset<S>(t, 0)) = make_uint2(w[0], w[1]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < S / 32; ++j)
+      *reinterpret_cast<uint4*>(out + slab_offset<S>(t, 16 * j)) =
+          make_uint4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]);
+  }
+  slab_scales[static_cast<int64_t>(r) * capacity + t] = static_cast<uint16_t>(sbits);
+}
+
+// Any alignment: S/8 lanes per token, 2-byte loads of the selected channels.
 template <int S, bool F16>
 __global__ __launch_bounds__(kThreads) void build_slab_kernel(
     const uint16_t* __restrict__ key, int64_t ksb, int64_t ksh, int64_t kst, int kv_heads,
@@ -203,17 +374,14 @@ __global__ __launch_bounds__(kThreads) void build_slab_kernel(
   const int32_t* idx = chan_idx + r * S + jj * 8;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    // channel ids come from qkv_int4_select_channels; clamping keeps a bad id in the row
     const int c = min(max(active ? idx[i] : 0, 0), head_dim - 1);
     x[i] = active ? half_to_f32<F16>(row[c]) : 0.0f;
   }
   float a = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) a = fmaxf(a, fabsf(x[i]));
-#pragma unroll
-  for (int m = 1; m < TPT; m <<= 1) a = fmaxf(a, shfl_xor(a, m));
-  uint32_t sbits;
-  uint32_t word = quantize8(x, a, &sbits);
+  const uint32_t sbits = group_scale(group_max<TPT>(a));
+  const uint32_t word = codes8(x, code_rcp(f16bits_to_f32(sbits)));
   if (active) {
     const int64_t tok = r * capacity + t;
     *reinterpret_cast<uint32_t*>(slab + r * capacity * (S / 2) + slab_offset<S>(t, 4 * jj)) = word;
@@ -329,15 +497,17 @@ QKV_EXPORT int qkv_int4_pack_k(const void* key, const int64_t* k_strides, int64_
     return fail(QKV_ERR_INVALID, "qkv_int4_pack_k: capacity must be a multiple of 64 and outputs 16-byte aligned");
   const int64_t ntok = t_end - t_begin;
   if (ntok == 0) return QKV_OK;
-  const int64_t total = batch * kv_heads * ntok * (head_dim / 8);
-  dim3 grid(static_cast<unsigned>(cdiv(total, kThreads)));
+  const int tpt_log2 = head_dim == 64 ? 3 : head_dim == 128 ? 4 : 5;
+  const int64_t tiles = cdiv(ntok, kPackIter * (kThreads >> tpt_log2));
+  if (batch * kv_heads * tiles > 0x7FFFFFFF) return fail(QKV_ERR_INVALID, "qkv_int4_pack_k: too many tokens");
+  dim3 grid(static_cast<unsigned>(batch * kv_heads * tiles));
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint16_t* k = static_cast<const uint16_t*>(key);
 #define QKV_PACK(GG, FF)                                                                              \
   pack_kernel<GG, FF><<<grid, kThreads, 0, st>>>(k, k_strides[0], k_strides[1], k_strides[2],        \
                                                  static_cast<int>(kv_heads), static_cast<int>(t_begin), \
-                                                 static_cast<int>(ntok), static_cast<int>(head_dim),  \
-                                                 packed, scales, capacity, total)
+                                                 static_cast<int>(t_end), tpt_log2,                   \
+                                                 static_cast<unsigned>(tiles), packed, scales, capacity)
   if (f16) {
     if (group == 32) QKV_PACK(32, true);
     else if (group == 64) QKV_PACK(64, true);
@@ -351,10 +521,17 @@ QKV_EXPORT int qkv_int4_pack_k(const void* key, const int64_t* k_strides, int64_
   return check_launch("qkv_int4_pack_k");
 }
 
-QKV_EXPORT int qkv_int4_select_channels(const uint8_t* packed, const uint16_t* scales, int64_t rows,
-                                        int64_t tokens, int64_t capacity, int64_t head_dim,
-                                        int64_t group, int64_t selected, uint64_t* stats,
-                                        int32_t* chan_idx, void* stream) {
+// Token chunks of the channel statistic: about 2048 workgroups over the rows,
+// chunks of at least 128 tokens (one round of four loads at D = 128) and at
+// most 128 a row, so that the partial sums stay a small share of the read.
+static int64_t stats_chunk(int64_t rows, int64_t tokens) {
+  const int64_t want = std::min<int64_t>(128, std::max<int64_t>(1, 2048 / rows));
+  return std::max<int64_t>(128, cdiv(cdiv(tokens, want), 128) * 128);
+}
+
+static int check_select(const uint8_t* packed, const uint16_t* scales, int64_t rows, int64_t tokens,
+                        int64_t capacity, int64_t head_dim, int64_t group, int64_t selected, const uint64_t* stats,
+                        const int32_t* chan_idx) {
   if (!packed || !scales || !stats || !chan_idx)
     return fail(QKV_ERR_INVALID, "qkv_int4_select_channels: null pointer");
   if (rows <= 0 || rows > 65535 || tokens <= 0 || tokens > capacity || tokens > (int64_t(1) << 20))
@@ -366,21 +543,57 @@ QKV_EXPORT int qkv_int4_select_channels(const uint8_t* packed, const uint16_t* s
   if (selected < 1 || selected > head_dim)
     return fail(QKV_ERR_INVALID, "qkv_int4_select_channels: selected must be in [1, head_dim]");
   if (capacity % 64) return fail(QKV_ERR_INVALID, "qkv_int4_select_channels: capacity must be a multiple of 64");
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t n = rows * head_dim;
-  zero_u64_kernel<<<static_cast<unsigned>(cdiv(n, kThreads)), kThreads, 0, st>>>(stats, n);
-  int rc = check_launch("qkv_int4_select_channels(zero)");
-  if (rc) return rc;
-  const int chunk = 4096;
+  return QKV_OK;
+}
+
+// The statistic and the selection; `part` (may be null) holds the chunks' sums.
+static int run_select(const uint8_t* packed, const uint16_t* scales, int64_t rows, int64_t tokens, int64_t capacity,
+                      int64_t head_dim, int64_t group, int64_t selected, uint64_t* part, uint64_t* stats,
+                      int32_t* chan_idx, hipStream_t st) {
+  const int64_t chunk = stats_chunk(rows, tokens);
   dim3 grid(static_cast<unsigned>(cdiv(tokens, chunk)), static_cast<unsigned>(rows));
+  if (!part) {
+    const int64_t n = rows * head_dim;
+    zero_u64_kernel<<<static_cast<unsigned>(cdiv(n, kThreads)), kThreads, 0, st>>>(stats, n);
+    if (int rc = check_launch("qkv_int4_select_channels(zero)")) return rc;
+  }
   channel_stats_kernel<<<grid, kThreads, 0, st>>>(packed, scales, static_cast<int>(tokens), capacity,
                                                   static_cast<int>(head_dim), static_cast<int>(group),
-                                                  chunk, stats);
-  rc = check_launch("qkv_int4_select_channels(stats)");
-  if (rc) return rc;
-  select_channels_kernel<<<static_cast<unsigned>(rows), 64, 0, st>>>(stats, static_cast<int>(head_dim),
-                                                                     static_cast<int>(selected), chan_idx);
+                                                  static_cast<int>(chunk), part, stats);
+  if (int rc = check_launch("qkv_int4_select_channels(stats)")) return rc;
+  select_channels_kernel<<<static_cast<unsigned>(rows), 1024, 0, st>>>(
+      part, part ? static_cast<int>(grid.x) : 0, stats, static_cast<int>(head_dim), static_cast<int>(selected),
+      chan_idx);
   return check_launch("qkv_int4_select_channels(select)");
+}
+
+QKV_EXPORT int qkv_int4_select_channels(const uint8_t* packed, const uint16_t* scales, int64_t rows,
+                                        int64_t tokens, int64_t capacity, int64_t head_dim,
+                                        int64_t group, int64_t selected, uint64_t* stats,
+                                        int32_t* chan_idx, void* stream) {
+  if (int rc = check_select(packed, scales, rows, tokens, capacity, head_dim, group, selected, stats, chan_idx))
+    return rc;
+  return run_select(packed, scales, rows, tokens, capacity, head_dim, group, selected, nullptr, stats, chan_idx,
+                    static_cast<hipStream_t>(stream));
+}
+
+QKV_EXPORT int64_t qkv_int4_select_channels_workspace_bytes(int64_t rows, int64_t tokens, int64_t head_dim) {
+  if (rows <= 0 || tokens <= 0 || head_dim <= 0) return -1;
+  return rows * cdiv(tokens, stats_chunk(rows, tokens)) * head_dim * 8;
+}
+
+QKV_EXPORT int qkv_int4_select_channels_ws(const uint8_t* packed, const uint16_t* scales, int64_t rows,
+                                           int64_t tokens, int64_t capacity, int64_t head_dim, int64_t group,
+                                           int64_t selected, uint64_t* stats, int32_t* chan_idx, void* workspace,
+                                           int64_t workspace_bytes, void* stream) {
+  if (int rc = check_select(packed, scales, rows, tokens, capacity, head_dim, group, selected, stats, chan_idx))
+    return rc;
+  const int64_t need = qkv_int4_select_channels_workspace_bytes(rows, tokens, head_dim);
+  if (!workspace || workspace_bytes < need || !aligned(workspace, 8))
+    return fail(QKV_ERR_INVALID, "qkv_int4_select_channels_ws: workspace needs %lld bytes (8-byte aligned), got %lld",
+                (long long)need, (long long)workspace_bytes);
+  return run_select(packed, scales, rows, tokens, capacity, head_dim, group, selected,
+                    static_cast<uint64_t*>(workspace), stats, chan_idx, static_cast<hipStream_t>(stream));
 }
 
 QKV_EXPORT int qkv_int4_build_slab(const void* key, const int64_t* k_strides, int64_t batch,
@@ -402,10 +615,39 @@ QKV_EXPORT int qkv_int4_build_slab(const void* key, const int64_t* k_strides, in
                 (long long)slab_tile_keys(static_cast<int>(selected)));
   const int64_t ntok = t_end - t_begin;
   if (ntok == 0) return QKV_OK;
-  const int64_t total = batch * kv_heads * ntok * (selected / 8);
-  dim3 grid(static_cast<unsigned>(cdiv(total, kThreads)));
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint16_t* k = static_cast<const uint16_t*>(key);
+  const int64_t tiles = cdiv(ntok, 64);
+  if (aligned(key, 16) && (k_strides[0] | k_strides[1] | k_strides[2]) % 8 == 0 &&
+      (head_dim == 64 || head_dim == 128 || head_dim == 256) && batch * kv_heads * tiles <= 0x7FFFFFFF) {
+    const unsigned rgrid = static_cast<unsigned>(batch * kv_heads * tiles);
+    auto launch = [&](auto sc, auto dc) {
+      constexpr int SS = decltype(sc)::value, DD = decltype(dc)::value;
+      if constexpr (SS <= DD) {
+        return with_half(f16, [&](auto fc) {
+          build_slab_rows_kernel<SS, DD, decltype(fc)::value><<<rgrid, 64, 0, st>>>(
+              k, k_strides[0], k_strides[1], k_strides[2], static_cast<int>(kv_heads), static_cast<int>(t_begin),
+              static_cast<int>(t_end), static_cast<unsigned>(tiles), chan_idx, slab, slab_scales, capacity);
+          return check_launch("qkv_int4_build_slab");
+        });
+      } else {
+        return fail(QKV_ERR_INVALID, "qkv_int4_build_slab: selected > head_dim");
+      }
+    };
+    auto with_d = [&](auto sc) {
+      if (head_dim == 64) return launch(sc, std::integral_constant<int, 64>{});
+      if (head_dim == 128) return launch(sc, std::integral_constant<int, 128>{});
+      return launch(sc, std::integral_constant<int, 256>{});
+    };
+    switch (selected) {
+      case 16: return with_d(std::integral_constant<int, 16>{});
+      case 32: return with_d(std::integral_constant<int, 32>{});
+      case 64: return with_d(std::integral_constant<int, 64>{});
+      default: return with_d(std::integral_constant<int, 128>{});
+    }
+  }
+  const int64_t total = batch * kv_heads * ntok * (selected / 8);
+  dim3 grid(static_cast<unsigned>(cdiv(total, kThreads)));
 #define QKV_SLAB(SS, FF)                                                                             \
   build_slab_kernel<SS, FF><<<grid, kThreads, 0, st>>>(k, k_strides[0], k_strides[1], k_strides[2], \
                                                        static_cast<int>(kv_heads), static_cast<int>(t_begin), \

@@ -108,9 +108,11 @@ def select_channels(packed: torch.Tensor, scales: torch.Tensor, tokens: int, gro
     stats = torch.empty((b, h, d), dtype=torch.int64, device=packed.device)
     chan = torch.empty((b, h, int(count)), dtype=torch.int32, device=packed.device)
     with _lib.on_device(packed.device):
-        _lib.check(lib.qkv_int4_select_channels(packed.data_ptr(), scales.data_ptr(), b * h, int(tokens), cap,
-                                                d, int(group), int(count), stats.data_ptr(), chan.data_ptr(),
-                                                _lib.stream_of(packed)))
+        need = lib.qkv_int4_select_channels_workspace_bytes(b * h, int(tokens), d)
+        ws = torch.empty(max(0, need) // 8, dtype=torch.int64, device=packed.device)
+        _lib.check(lib.qkv_int4_select_channels_ws(packed.data_ptr(), scales.data_ptr(), b * h, int(tokens), cap,
+                                                   d, int(group), int(count), stats.data_ptr(), chan.data_ptr(),
+                                                   ws.data_ptr(), need, _lib.stream_of(packed)))
     return chan, stats
 
 
