@@ -49,7 +49,7 @@ constexpr int kMaxScan = kRerankNT * 40;   // scanned tokens per row in one work
 __device__ void rank_dims(const float* q_s, int count, int* sel_idx, float* sel_q) {
   __shared__ __attribute__((aligned(16))) uint64_t key_s[kHD];
   __syncthreads();
-  rank_dims128(q_s, key_s, kHD, count, sel_idx, sel_q);
+  rank_dims128<QKV_DTYPE_BF16>(q_s, key_s, kHD, count, sel_idx, sel_q);   // (16-bit queries)
 }
 
 // The 16-bit pattern of v, a value of the dtype (exact).

@@ -66,7 +66,7 @@ __global__ __launch_bounds__(kLagNT) void lag_flags_kernel(
   __syncthreads();
   // the step's top-|q| dims, descending |q| with ties to the lower dim, and
   // q at them (EV:4026-4027, recorded at EV:4384-4393)
-  rank_dims128(q_s, key_s, head_dim, count, sel_idx, sel_q);
+  rank_dims128<DT>(q_s, key_s, head_dim, count, sel_idx, sel_q);
   for (int s = tid; s < count; s += kLagNT) {
     dims_out[static_cast<int64_t>(row) * count + s] = sel_idx[s];
     vals_out[static_cast<int64_t>(row) * count + s] = sel_q[s];
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(kLagNT) void lag_ess_kernel(
   for (int d = tid; d < 128; d += kLagNT) q_s[d] = d < head_dim ? Elem<DT>::load(q_row + d) : 0.f;
   __syncthreads();
   if (split == 0) {   // uniform: the row's top-|q| dims, as lag_flags_kernel records them
-    rank_dims128(q_s, key_s, head_dim, count, sel_idx, sel_q);
+    rank_dims128<DT>(q_s, key_s, head_dim, count, sel_idx, sel_q);
     for (int s = tid; s < count; s += kLagNT) {
       dims_out[static_cast<int64_t>(row) * count + s] = sel_idx[s];
       vals_out[static_cast<int64_t>(row) * count + s] = sel_q[s];

@@ -63,53 +63,78 @@ __device__ void select_dims(const typename Elem<DT>::T* q_row, int head_dim, int
 }
 
 // The same order for head_dim <= 128 dims whose query values sit in LDS
-// (q_s), with one 64-bit key per dim: the bits of |q_d| (for non-negative
+// (q_s), with one integer key per dim: the bits of |q_d| (for non-negative
 // floats the integer order is the numeric order) above 255 - d, so that
 // "larger |q|, or equal |q| and lower dim" is one unsigned compare and
-// rank(d) is the number of keys above d's.  The 128 keys (dims past head_dim
-// pad with 0, under every real key) are read back by broadcast 16-byte LDS
-// loads.  key_s: 128 LDS words of 8 bytes.  Every thread calls it; it begins
-// after a barrier that published q_s and ends with one.
+// rank(d) is the number of keys above d's.  A widened bf16 or fp16 leaves at
+// least 13 low bits of the fp32 pattern zero, so its key fits 32 bits (64-bit
+// compares issue at a fraction of the 32-bit rate); fp32 takes 64.  The 128
+// keys (dims past head_dim pad with 0, under every real key) are read back by
+// broadcast 16-byte LDS loads, every 128 threads of the workgroup taking a
+// share of them.  key_s: 128 LDS words of 8 bytes.  Every thread of a
+// workgroup of at least 128 calls it; it begins after a barrier that
+// published q_s and ends with one.
+template <int DT>
 __device__ inline void rank_dims128(const float* q_s, uint64_t* key_s, int head_dim, int count, int* sel_idx,
                                     float* sel_q) {
+  using K = std::conditional_t<DT == QKV_DTYPE_FP32, uint64_t, uint32_t>;
   const int tid = threadIdx.x;
+  K* key = reinterpret_cast<K*>(key_s);
+  __shared__ int rank_s[128];
   for (int s = tid; s < count; s += blockDim.x) {   // valid even for a NaN query
     sel_idx[s] = 0;
     sel_q[s] = q_s[0];
   }
-  for (int d = tid; d < 128; d += blockDim.x)
-    key_s[d] = d < head_dim ? (static_cast<uint64_t>(__float_as_uint(q_s[d]) & 0x7FFFFFFFu) << 8) |
-                                  static_cast<uint64_t>(255 - d)
-                            : 0ull;
+  if (tid < 128) {
+    const uint32_t a = tid < head_dim ? __float_as_uint(q_s[tid]) & 0x7FFFFFFFu : 0u;
+    const uint32_t low = tid < head_dim ? 255u - tid : 0u;
+    if constexpr (DT == QKV_DTYPE_FP32) key[tid] = (static_cast<uint64_t>(a) << 8) | low;
+    else key[tid] = a | low;
+    rank_s[tid] = 0;
+  }
   __syncthreads();
-  for (int d = tid; d < head_dim; d += blockDim.x) {
-    const uint64_t own = key_s[d];
+  const int parts = blockDim.x >> 7;           // shares of the 128 keys (a power of two up to 8)
+  if (tid < parts * 128) {
+    const int d = tid & 127, per = 128 / parts, e0 = (tid >> 7) * per;
+    const K own = key[d];
     int rank = 0;
+    constexpr int kStep = 16 / sizeof(K);
 #pragma unroll 8   // (eight 16-byte reads in flight; a full unroll holds all 128 keys in registers)
-    for (int e = 0; e < 128; e += 2) {
-      const ulonglong2 c = *reinterpret_cast<const ulonglong2*>(key_s + e);
-      rank += (c.x > own ? 1 : 0) + (c.y > own ? 1 : 0);
+    for (int e = e0; e < e0 + per; e += kStep) {
+      if constexpr (DT == QKV_DTYPE_FP32) {
+        const ulonglong2 c = *reinterpret_cast<const ulonglong2*>(key + e);
+        rank += (c.x > own ? 1 : 0) + (c.y > own ? 1 : 0);
+      } else {
+        const uint4 c = *reinterpret_cast<const uint4*>(key + e);
+        rank += (c.x > own ? 1 : 0) + (c.y > own ? 1 : 0) + (c.z > own ? 1 : 0) + (c.w > own ? 1 : 0);
+      }
     }
-    if (rank < count) {
-      sel_idx[rank] = d;
-      sel_q[rank] = q_s[d];
-    }
+    if (rank) atomicAdd(&rank_s[d], rank);
+  }
+  __syncthreads();
+  if (tid < head_dim && rank_s[tid] < count) {
+    sel_idx[rank_s[tid]] = tid;
+    sel_q[rank_s[tid]] = q_s[tid];
   }
   __syncthreads();
 }
 
-// Eight consecutive elements at p as fp32 (p 16-byte aligned).
+// Eight consecutive elements at p as fp32, at any element alignment (gfx950
+// global loads take unaligned addresses; a 16-byte load that crosses a line
+// costs that line).
 template <int DT>
 __device__ __forceinline__ void load8(const typename Elem<DT>::T* p, float (&v)[8]) {
   if constexpr (DT == QKV_DTYPE_FP32) {
-    const uint4 a = *reinterpret_cast<const uint4*>(p);
-    const uint4 c = *reinterpret_cast<const uint4*>(p + 4);
+    uint4 a, c;
+    __builtin_memcpy(&a, p, 16);
+    __builtin_memcpy(&c, p + 4, 16);
     v[0] = __uint_as_float(a.x); v[1] = __uint_as_float(a.y);
     v[2] = __uint_as_float(a.z); v[3] = __uint_as_float(a.w);
     v[4] = __uint_as_float(c.x); v[5] = __uint_as_float(c.y);
     v[6] = __uint_as_float(c.z); v[7] = __uint_as_float(c.w);
   } else {
-    const uint4 a = *reinterpret_cast<const uint4*>(p);
+    uint4 a;
+    __builtin_memcpy(&a, p, 16);
     const uint32_t w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

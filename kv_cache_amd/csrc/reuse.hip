@@ -42,7 +42,10 @@ constexpr int kMaskTile = 4096;   // tokens per workgroup in reuse_mask_kernel
 // ---------------------------------------------------------------------------
 // Partial scores: out[r, t] = sum_s q[d_s] * K[d_s, t] over the row's
 // top-|q| dims d_s in selection order (QK:63-96 on the dim-major copy of
-// EV:2018-2042; dims chosen as QK:120-145).  Eight tokens per thread.
+// EV:2018-2042; dims chosen as QK:120-145).  Eight tokens per thread, one
+// 16-byte load per dim at any alignment: a copy whose rows hold an odd
+// number of tokens reads at the same rate (128 rows x 16410 tokens, S = 8:
+// 28.7 us with element loads there, 12.8 us now).
 // HIST: each score's top 12 order-preserving bits (the first radix digit of
 // the candidate selection, kCandBins bins) are also counted into
 // hist[row * kCandBins + digit], through a workgroup histogram in LDS and
@@ -59,7 +62,7 @@ template <int DT, bool HIST = false>
 __global__ __launch_bounds__(kPartNT) void reuse_partial_kernel(
     const typename Elem<DT>::T* __restrict__ query, const typename Elem<DT>::T* __restrict__ kdm,
     int q_heads, int group, int history, int head_dim, int count, int64_t sb, int64_t sh, int64_t sd,
-    bool vec, float* __restrict__ out, int64_t out_ld, const uint8_t* __restrict__ gate, int gate_refresh,
+    float* __restrict__ out, int64_t out_ld, const uint8_t* __restrict__ gate, int gate_refresh,
     int gate_rows, int* __restrict__ hist = nullptr) {
   using E = typename Elem<DT>::T;
   __shared__ int hist_s[HIST ? kCandBins : 1];
@@ -81,7 +84,7 @@ __global__ __launch_bounds__(kPartNT) void reuse_partial_kernel(
   for (int d = tid; d < head_dim; d += kPartNT) q_s[d] = Elem<DT>::load(q_row + d);
   __syncthreads();
   if (head_dim <= 128) {   // uniform
-    rank_dims128(q_s, key_s, head_dim, count, sel_idx, sel_q);
+    rank_dims128<DT>(q_s, key_s, head_dim, count, sel_idx, sel_q);
   } else {
     for (int s = tid; s < count; s += kPartNT) {   // valid even for a NaN query
       sel_idx[s] = 0;
@@ -113,7 +116,7 @@ __global__ __launch_bounds__(kPartNT) void reuse_partial_kernel(
   for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
   if (nt == 0) {
     // (HIST: a thread past the row still takes part in the barriers below)
-  } else if (vec && nt == 8) {
+  } else if (nt == 8) {
     // eight dims' loads in flight at once (clamped, in bounds), then the
     // products added in selection order
     for (int s0 = 0; s0 < count; s0 += 8) {
@@ -132,7 +135,7 @@ __global__ __launch_bounds__(kPartNT) void reuse_partial_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = acc[i];
   } else {
-    // the row's last n < 8 tokens (or an unaligned copy): the same order,
+    // the row's last n < 8 tokens: the same order,
     // every load in flight at once at clamped in-row addresses, then only
     // the n tokens stored (a load-then-add loop over runtime n waits for
     // each load in turn)
@@ -1086,7 +1089,7 @@ __global__ __launch_bounds__(kWideNT) void reuse_cand_slices_kernel(
 }
 
 // The step's candidates in one launch (rows of at most kWideMax history
-// tokens, head_dim <= 128, a 16-byte aligned dim-major copy): one 1024-thread
+// tokens, head_dim <= 128): one 1024-thread
 // workgroup per row forms the row's partial scores as reuse_partial_kernel
 // does (eight consecutive tokens per thread and chunk, NCH chunks, the same
 // loads and summation order), writes them, counts their first radix digit
@@ -1122,7 +1125,7 @@ __global__ __launch_bounds__(kWideNT) void reuse_candidates_kernel(
 #pragma unroll
   for (int j = 0; j < WS::NB / kWideNT; ++j) wsh.hist[0][tid + kWideNT * j] = 0;
   __syncthreads();
-  rank_dims128(q_s, key_s, head_dim, count, sel_idx, sel_q);   // (ends with a barrier)
+  rank_dims128<DT>(q_s, key_s, head_dim, count, sel_idx, sel_q);   // (ends with a barrier)
 
   WS ws;
   int ninf = 0;
@@ -1908,14 +1911,12 @@ template <int DT> struct RunReusePartial {
                  int64_t T, int64_t D, int count, float* out, int64_t out_ld, hipStream_t st,
                  const uint8_t* gate = nullptr, int gate_refresh = 0, int* hist = nullptr) {
     using E = typename Elem<DT>::T;
-    const int64_t ev = DT == QKV_DTYPE_FP32 ? 4 : 8;   // elements per 16 bytes
-    const bool vec = aligned(kdm, 16) && ks[0] % ev == 0 && ks[1] % ev == 0 && ks[2] % ev == 0;
     dim3 grid(static_cast<unsigned>(cdiv(T, 8 * kPartNT)), static_cast<unsigned>(B * Hq));
 #define QKV_REUSE_PARTIAL(HH)                                                                                  \
   reuse_partial_kernel<DT, HH><<<grid, kPartNT, 0, st>>>(static_cast<const E*>(q), static_cast<const E*>(kdm),     \
                                                      static_cast<int>(Hq), static_cast<int>(Hq / Hkv),         \
                                                      static_cast<int>(T), static_cast<int>(D), count, ks[0],   \
-                                                     ks[1], ks[2], vec, out, out_ld, gate, gate_refresh,       \
+                                                     ks[1], ks[2], out, out_ld, gate, gate_refresh,            \
                                                      static_cast<int>(B * Hq), hist)
     if (hist) QKV_REUSE_PARTIAL(true);
     else QKV_REUSE_PARTIAL(false);
@@ -2090,14 +2091,12 @@ template <int DT> struct RunCandidates {
                  hipStream_t st, const uint8_t* gate, int refresh, uint64_t* bits = nullptr,
                  int64_t bits_ld = 0, const CandSplit& split = CandSplit{}) {
     using E = typename Elem<DT>::T;
-    const int64_t ev = DT == QKV_DTYPE_FP32 ? 4 : 8;   // elements per 16 bytes
-    const bool vec = aligned(kdm, 16) && ks[0] % ev == 0 && ks[1] % ev == 0 && ks[2] % ev == 0;
     const int64_t rows = B * Hq;
     // One launch pays off once the rows fill the GPU: measured at 32768 tokens,
     // 32 rows took 27.1 us fused against 26.3 us for the two launches (and more
     // inside a decode step, where the copy's rows come from HBM), 128 rows 31.1
     // against 41.1 us, 256 rows 40.4 against 58.1 us.
-    if (vec && T <= kWideMax && D <= 128 && rows >= kFusedCandRows) {
+    if (T <= kWideMax && D <= 128 && rows >= kFusedCandRows) {
       auto launch = [&](auto nch) {
         reuse_candidates_kernel<DT, decltype(nch)::value><<<static_cast<unsigned>(rows), kWideNT, 0, st>>>(
             static_cast<const E*>(q), static_cast<const E*>(kdm), static_cast<int>(Hq), static_cast<int>(Hq / Hkv),
