@@ -89,6 +89,12 @@ int qkv_partial_scores_dim_major(const void* query, const void* key_dim_major,
                                  int64_t batch, int64_t heads, int64_t keys, int64_t head_dim,
                                  int64_t selected, const int64_t* kdm_strides, void* stream);
 
+/* ids[i] = indices[i] where valid[i] is not 0 and 0 <= indices[i] < keys,
+ * else -1: the int32 lists qkv_token_attention reads from the int64 / bool
+ * lists of QK:569-638. */
+int qkv_token_ids(const int64_t* indices, const uint8_t* valid, int64_t count, int64_t keys,
+                  int32_t* ids, void* stream);
+
 /* Replaces qabs_candidate_full_scores_forward (QK:506-567, kernel
  * QK:160-216, Python candidate_full_scores QK:668-691).
  * Masks are uint8 [B,H,T] contiguous; previous / previous_final may be NULL.

@@ -40,6 +40,7 @@ _PROTOTYPES = {
                                          _P(_i64), _i64, _i64, _f32, _vp]),
     "qkv_final_attention": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _i64,
                                    _f32, _vp]),
+    "qkv_token_ids": (_i32, [_vp, _vp, _i64, _i64, _vp, _vp]),
     "qkv_int4_pack_k": (_i32, [_vp, _P(_i64), _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _i64, _i32, _vp]),
     "qkv_int4_select_channels": (_i32, [_vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp]),
     "qkv_int4_select_channels_workspace_bytes": (_i64, [_i64, _i64, _i64]),

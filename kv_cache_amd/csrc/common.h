@@ -222,6 +222,13 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
+// 16 bytes at any alignment (gfx950 global loads take unaligned addresses).
+__device__ __forceinline__ uint4 load16u(const void* p) {
+  u32x4_t a;
+  __builtin_memcpy(&a, p, 16);
+  return make_uint4(a.x, a.y, a.z, a.w);
+}
+
 // DPP move within rows of 16 lanes (quad_perm, row_shl/shr, row mirrors ...),
 // every row and bank enabled.
 template <int DPP>

@@ -125,16 +125,13 @@ __device__ inline void rank_dims128(const float* q_s, uint64_t* key_s, int head_
 template <int DT>
 __device__ __forceinline__ void load8(const typename Elem<DT>::T* p, float (&v)[8]) {
   if constexpr (DT == QKV_DTYPE_FP32) {
-    uint4 a, c;
-    __builtin_memcpy(&a, p, 16);
-    __builtin_memcpy(&c, p + 4, 16);
+    const uint4 a = load16u(p), c = load16u(p + 4);
     v[0] = __uint_as_float(a.x); v[1] = __uint_as_float(a.y);
     v[2] = __uint_as_float(a.z); v[3] = __uint_as_float(a.w);
     v[4] = __uint_as_float(c.x); v[5] = __uint_as_float(c.y);
     v[6] = __uint_as_float(c.z); v[7] = __uint_as_float(c.w);
   } else {
-    uint4 a;
-    __builtin_memcpy(&a, p, 16);
+    const uint4 a = load16u(p);
     const uint32_t w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

@@ -33,6 +33,64 @@ __global__ __launch_bounds__(kTile) void partial_scores_kernel(
   out[static_cast<int64_t>(row) * keys + t] = acc;
 }
 
+// The same for head size 128 with contiguous channels (any alignment): a
+// wave takes kRowTok tokens, loads their whole rows with 16-byte loads, all
+// in flight before the dims are ranked, stages them in LDS (every 128-byte
+// line of a row holds selected channels, so nothing is read in vain) and
+// then scores one token per lane in the selection order.  LDS rows are 16
+// bytes longer than K's, so a read's lanes spread over the banks.
+// 32 heads x 8190 tokens, 16 dims, bf16 (67 MB of K): 31.8 us with one
+// 2-byte load per lane and dim, 15.2 us now.
+constexpr int kRowWaves = 2;
+template <int DT>
+__global__ __launch_bounds__(64 * kRowWaves) void partial_scores_rows_kernel(
+    const typename Elem<DT>::T* __restrict__ query, const typename Elem<DT>::T* __restrict__ key,
+    float* __restrict__ out, int heads, int keys, int count, int64_t ksb, int64_t ksh, int64_t kst) {
+  using E = typename Elem<DT>::T;
+  constexpr int kEl = 16 / static_cast<int>(sizeof(E));   // elements per 16 bytes
+  constexpr int kPieces = 128 / kEl;                      // 16-byte pieces of a row: 16 or 32
+  constexpr int kRowTok = 1024 / kPieces;                 // tokens of a wave: 64, or 32 for fp32
+  constexpr int kTok = 64 / kPieces;                      // tokens per load of the wave
+  __shared__ uint4 rows[kRowWaves][kRowTok * (kPieces + 1)];
+  __shared__ __attribute__((aligned(16))) uint64_t key_s[128];
+  __shared__ float q_s[128];
+  __shared__ int sel_idx[kMaxDims];
+  __shared__ float sel_q[kMaxDims];
+  const int row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int b = row / heads, h = row - b * heads;
+  const int t0 = (blockIdx.x * kRowWaves + wave) * kRowTok;
+  const int piece = lane % kPieces, tl = lane / kPieces;
+  const E* base = key + b * ksb + h * ksh + piece * kEl;
+  const float q0 = Elem<DT>::load(query + static_cast<int64_t>(row) * 128 + tid);
+  uint4 raw[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i)   // (tokens past the row: its last one again)
+    raw[i] = load16u(base + static_cast<int64_t>(min(t0 + i * kTok + tl, keys - 1)) * kst);
+  q_s[tid] = q0;
+  __syncthreads();
+  rank_dims128<DT>(q_s, key_s, 128, count, sel_idx, sel_q);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) rows[wave][(i * kTok + tl) * (kPieces + 1) + piece] = raw[i];
+  __syncthreads();
+  const int t = t0 + lane;
+  if (lane >= kRowTok || t >= keys) return;
+  const E* own = reinterpret_cast<const E*>(&rows[wave][lane * (kPieces + 1)]);
+  float acc = 0.0f;
+  for (int s0 = 0; s0 < count; s0 += 8) {   // eight reads in flight, added in selection order
+    float v[8], qv[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int s = min(s0 + j, count - 1);
+      v[j] = Elem<DT>::load(own + sel_idx[s]);
+      qv[j] = sel_q[s];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (s0 + j < count) acc = acc + qv[j] * v[j];
+  }
+  out[static_cast<int64_t>(row) * keys + t] = acc;
+}
+
 template <int DT>
 __global__ __launch_bounds__(kTile) void partial_scores_dim_major_kernel(
     const typename Elem<DT>::T* __restrict__ query, const typename Elem<DT>::T* __restrict__ kdm,
@@ -168,6 +226,14 @@ template <int DT> struct RunPartial {
   static int run(const void* q, const void* k, float* out, int64_t B, int64_t H, int64_t T,
                  int64_t D, const int64_t* ks, int count, hipStream_t st) {
     using E = typename Elem<DT>::T;
+    if (D == 128 && ks[3] == 1) {
+      constexpr int tok = kRowWaves * (DT == QKV_DTYPE_FP32 ? 32 : 64);
+      dim3 rgrid(static_cast<unsigned>(cdiv(T, tok)), static_cast<unsigned>(B * H));
+      partial_scores_rows_kernel<DT><<<rgrid, 64 * kRowWaves, 0, st>>>(
+          static_cast<const E*>(q), static_cast<const E*>(k), out, static_cast<int>(H), static_cast<int>(T), count,
+          ks[0], ks[1], ks[2]);
+      return check_launch("qkv_partial_scores");
+    }
     dim3 grid(static_cast<unsigned>(cdiv(T, kTile)), static_cast<unsigned>(B * H));
     partial_scores_kernel<DT><<<grid, kTile, 0, st>>>(
         static_cast<const E*>(q), static_cast<const E*>(k), out, static_cast<int>(H),
@@ -224,10 +290,35 @@ int check_common(const void* q, const void* k, int64_t B, int64_t H, int64_t T, 
   return QKV_OK;
 }
 
+// One int32 id per int64 index: -1 where it is not valid or lies outside the keys.
+__global__ __launch_bounds__(kTile) void token_ids_kernel(const int64_t* __restrict__ indices,
+                                                          const uint8_t* __restrict__ valid, int64_t n,
+                                                          int64_t keys, int32_t* __restrict__ ids) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kTile + threadIdx.x;
+  if (i >= n) return;
+  const int64_t t = indices[i];
+  ids[i] = valid[i] != 0 && t >= 0 && t < keys ? static_cast<int32_t>(t) : -1;
+}
+
 }  // namespace
+
+int union_scores(int dtype, const void* query, const void* key, const int64_t* k_strides, int64_t batch,
+                 int64_t heads, int64_t keys, int64_t head_dim, const uint8_t* current, const uint8_t* previous,
+                 const uint8_t* previous_final, int sink, int recent, float scaling, float* out, hipStream_t st);
 }  // namespace qkv
 
 using namespace qkv;
+
+QKV_EXPORT int qkv_token_ids(const int64_t* indices, const uint8_t* valid, int64_t count, int64_t keys, int32_t* ids,
+                             void* stream) {
+  if (!indices || !valid || !ids) return fail(QKV_ERR_INVALID, "qkv_token_ids: null pointer");
+  if (count < 0 || keys < 0 || keys >= (int64_t(1) << 31) || cdiv(count, kTile) > 0x7FFFFFFF)
+    return fail(QKV_ERR_INVALID, "qkv_token_ids: bad sizes");
+  if (count == 0) return QKV_OK;
+  token_ids_kernel<<<static_cast<unsigned>(cdiv(count, kTile)), kTile, 0, static_cast<hipStream_t>(stream)>>>(
+      indices, valid, count, keys, ids);
+  return check_launch("qkv_token_ids");
+}
 
 QKV_EXPORT int qkv_partial_scores(const void* query, const void* key, float* out, int dtype,
                                   int64_t batch, int64_t heads, int64_t keys, int64_t head_dim,
@@ -275,6 +366,12 @@ QKV_EXPORT int qkv_candidate_full_scores(const void* query, const void* key, con
   if (keys == 0) return QKV_OK;
   int sink = static_cast<int>(std::min<int64_t>(std::max<int64_t>(protect_sink, 0), keys));
   int recent = static_cast<int>(std::min<int64_t>(std::max<int64_t>(protect_recent, 0), keys));
+  // contiguous channels: the reuse step's union scores (the selected tokens
+  // compacted, so that no lane waits for its unselected neighbours; 32 heads
+  // x 8190 tokens with 21% selected, bf16: 21.2 us one token per lane, 8.6 us so)
+  if (k_strides[3] == 1)
+    return union_scores(dtype, query, key, k_strides, batch, heads, keys, head_dim, current, previous,
+                        previous_final, sink, recent, scaling, out, static_cast<hipStream_t>(stream));
   return dispatch_dtype<RunCandidate>(dtype, query, key, current, previous, previous_final, out,
                                       batch, heads, keys, head_dim, k_strides, sink, recent,
                                       scaling, static_cast<hipStream_t>(stream));

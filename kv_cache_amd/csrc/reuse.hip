@@ -327,14 +327,16 @@ __global__ __launch_bounds__(kRT) void sample_mask_kernel(const float* __restric
 // registers are held to five waves per SIMD so that a row's 33 workgroups
 // times 32 rows are resident together (at three, a second batch waited).
 // BITS: the three masks are bitsets (64 positions per uint64 word, mask_ld
-// in words) instead of byte masks.
+// in words) instead of byte masks.  Byte masks: positions below `sink` and
+// from `recent_start` on are scored as well (QK:160-216's protected ranges;
+// 0 and the history for none).
 // ---------------------------------------------------------------------------
 template <int DT, int DFIX, bool BITS>
 __global__ __launch_bounds__(kScoreNT) __attribute__((amdgpu_waves_per_eu(5))) void reuse_scores_kernel(
     const typename Elem<DT>::T* __restrict__ query, const typename Elem<DT>::T* __restrict__ key,
     int q_heads, int group, int history, int head_dim, int64_t sb, int64_t sh, int64_t st, bool kvec,
     const uint8_t* __restrict__ cur, const uint8_t* __restrict__ prev, const uint8_t* __restrict__ fin,
-    int64_t mask_ld, bool mvec, float scaling, float* __restrict__ out, int64_t out_ld,
+    int64_t mask_ld, int sink, int recent_start, float scaling, float* __restrict__ out, int64_t out_ld,
     float* __restrict__ cscore, int32_t* __restrict__ ctok, int32_t* __restrict__ ccnt, int64_t c_ld) {
   using E = typename Elem<DT>::T;
   __shared__ __attribute__((aligned(16))) float q_s[512];
@@ -364,14 +366,16 @@ __global__ __launch_bounds__(kScoreNT) __attribute__((amdgpu_waves_per_eu(5))) v
       const int n = min(4, history - t0);
       bits = static_cast<uint32_t>(u >> (t0 & 63)) & ((1u << n) - 1u);
     }
-  } else if (mvec && t0 + 4 <= history) {
-    uint32_t u = *reinterpret_cast<const uint32_t*>(cur + moff);
-    if (prev) u |= *reinterpret_cast<const uint32_t*>(prev + moff);
-    if (fin) u |= *reinterpret_cast<const uint32_t*>(fin + moff);
+  } else if (t0 + 4 <= history) {   // (4-byte loads at any alignment)
+    uint32_t u, p = 0, f = 0;
+    __builtin_memcpy(&u, cur + moff, 4);
+    if (prev) __builtin_memcpy(&p, prev + moff, 4);
+    if (fin) __builtin_memcpy(&f, fin + moff, 4);
+    u |= p | f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) bits |= static_cast<uint32_t>(((u >> (8 * i)) & 0xFFu) != 0) << i;
   } else if (t0 < history) {
-    // the row's last few positions (or unaligned masks): every byte load in
+    // the row's last few positions: every byte load in
     // flight at once at clamped in-row positions, then the positions past
     // the row dropped (short-circuit loads would wait for one another)
     const int n = min(4, history - t0);
@@ -385,6 +389,11 @@ __global__ __launch_bounds__(kScoreNT) __attribute__((amdgpu_waves_per_eu(5))) v
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) bits |= static_cast<uint32_t>(i < n && (c[i] | p[i] | f[i]) != 0) << i;
+  }
+  if (!BITS && (t0 < sink || t0 + 4 > recent_start)) {   // candidate_full_scores' protected ranges
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      bits |= static_cast<uint32_t>(t0 + i < history && (t0 + i < sink || t0 + i >= recent_start)) << i;
   }
   if (tid < head_dim) q_s[tid] = q0;
   for (int d = tid + kScoreNT; d < head_dim; d += kScoreNT) q_s[d] = Elem<DT>::load(q_row + d);
@@ -1929,19 +1938,19 @@ template <int DT> struct RunReuseScores {
   static int run(const void* q, const void* k, const int64_t* ks, int64_t B, int64_t Hq, int64_t Hkv, int64_t T,
                  int64_t D, const uint8_t* cur, const uint8_t* prev, const uint8_t* fin, int64_t mask_ld,
                  float scaling, float* out, int64_t out_ld, float* cscore, int32_t* ctok, int32_t* ccnt,
-                 int64_t c_ld, hipStream_t st, bool bitsets = false) {
+                 int64_t c_ld, hipStream_t st, bool bitsets = false, int sink = 0, int recent = 0) {
     using E = typename Elem<DT>::T;
     const int64_t ev = DT == QKV_DTYPE_FP32 ? 4 : 8;
     const bool kvec = ks[3] == 1 && D % 8 == 0 && aligned(k, 16) && ks[0] % ev == 0 && ks[1] % ev == 0 &&
                       ks[2] % ev == 0;
-    const bool mvec = mask_ld % 4 == 0 && aligned(cur, 4) && (!prev || aligned(prev, 4)) && (!fin || aligned(fin, 4));
     dim3 grid(static_cast<unsigned>(cdiv(T, kScoreTile)), static_cast<unsigned>(B * Hq));
     if (ks[3] != 1) return fail(QKV_ERR_UNSUPPORTED, "qkv_reuse_select: K channels must be contiguous");
 #define QKV_REUSE_SCORES(DF, BB)                                                                               \
   reuse_scores_kernel<DT, DF, BB><<<grid, kScoreNT, 0, st>>>(static_cast<const E*>(q), static_cast<const E*>(k),    \
                                                         static_cast<int>(Hq), static_cast<int>(Hq / Hkv),      \
                                                         static_cast<int>(T), static_cast<int>(D), ks[0], ks[1], \
-                                                        ks[2], kvec, cur, prev, fin, mask_ld, mvec, scaling, out, \
+                                                        ks[2], kvec, cur, prev, fin, mask_ld, sink,             \
+                                                        static_cast<int>(T) - recent, scaling, out,             \
                                                         out_ld, cscore, ctok, ccnt, c_ld)
     if (bitsets) {
       if (kvec && D == 128) QKV_REUSE_SCORES(128, true);
@@ -2128,6 +2137,16 @@ template <int DT> struct RunCandidates {
 };
 
 }  // namespace
+
+// qkv_candidate_full_scores for contiguous channels: byte masks [rows, keys].
+int union_scores(int dtype, const void* query, const void* key, const int64_t* k_strides, int64_t batch,
+                 int64_t heads, int64_t keys, int64_t head_dim, const uint8_t* current, const uint8_t* previous,
+                 const uint8_t* previous_final, int sink, int recent, float scaling, float* out, hipStream_t st) {
+  return dispatch_dtype<RunReuseScores>(dtype, query, key, k_strides, batch, heads, heads, keys, head_dim, current,
+                                        previous, previous_final, keys, scaling, out, keys, nullptr, nullptr, nullptr,
+                                        int64_t{0}, st, false, sink, recent);
+}
+
 }  // namespace qkv
 
 using namespace qkv;

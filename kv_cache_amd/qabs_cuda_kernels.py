@@ -189,9 +189,11 @@ def final_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
         # G = 1 on these head-expanded K/V), the invalid and out-of-range entries
         # as skipped ids; a row with none valid gives 0, as QK:388, 404 do
         with _lib.on_device(q.device):
-            # ids outside [0, t) are skipped (int64 values clamped first so none wraps)
-            keep = val if val.dtype == torch.bool else val != 0
-            ids = torch.where(keep, idx.clamp(-1, t), -1).to(torch.int32).view(b * h, n)
+            if val.dtype not in (torch.bool, torch.uint8):
+                val = val != 0
+            ids = torch.empty((b * h, n), dtype=torch.int32, device=q.device)   # -1: skipped
+            _lib.check(lib.qkv_token_ids(idx.data_ptr(), val.data_ptr(), b * h * n, t, ids.data_ptr(),
+                                         _lib.stream_of(q)))
             ws = _token_attention_workspace(q.device, ws_bytes)
             out = torch.empty((b, h, d), dtype=q.dtype, device=q.device)
             _lib.check(lib.qkv_token_attention(
