@@ -1833,6 +1833,22 @@ int with_wide_vpl(int64_t n, F&& f) {
   return f(std::integral_constant<int, 40>{});
 }
 
+// The same in finer steps, for kernels that always work on the whole row: a
+// wave owns 64 * VPL consecutive positions, so a row a little longer than a
+// coarse step would leave half the workgroup's waves without keys and give
+// the others twice as many.
+template <typename F>
+int with_wide_vpl_fine(int64_t n, F&& f) {
+  if (n <= 4 * kWideNT) return f(std::integral_constant<int, 4>{});
+  if (n <= 8 * kWideNT) return f(std::integral_constant<int, 8>{});
+  if (n <= 12 * kWideNT) return f(std::integral_constant<int, 12>{});
+  if (n <= 16 * kWideNT) return f(std::integral_constant<int, 16>{});
+  if (n <= 20 * kWideNT) return f(std::integral_constant<int, 20>{});
+  if (n <= 24 * kWideNT) return f(std::integral_constant<int, 24>{});
+  if (n <= 28 * kWideNT) return f(std::integral_constant<int, 28>{});
+  return with_wide_vpl(n, f);
+}
+
 // ---------------------------------------------------------------------------
 // Dim-major copy of K: kdm[b, j, d, t] = K[b, j, t, d] for t in [t0, t1),
 // through a 32-token LDS tile (coalesced on both sides).
@@ -1991,7 +2007,7 @@ int threshold_mask_impl(const char* what, const float* values, int64_t rows, int
                         hipStream_t st, const uint8_t* gate = nullptr, int gate_refresh = 0,
                         uint64_t* bits = nullptr, int64_t bits_ld = 0) {
   if (n <= kWideMax) {   // (rows past the one-workgroup length are selected whatever the gate says)
-    return with_wide_vpl(n, [&](auto vpl) {
+    return with_wide_vpl_fine(n, [&](auto vpl) {
       reuse_mask_wide_kernel<decltype(vpl)::value><<<static_cast<unsigned>(rows), kWideNT, 0, st>>>(
           values, ld, static_cast<int>(n), static_cast<int>(k), mask, mask_ld, thr_out, gate, gate_refresh,
           static_cast<int>(rows), bits, bits_ld);
@@ -2357,7 +2373,7 @@ QKV_EXPORT int qkv_qabs_candidate_select(const float* scores, int64_t rows, int6
                 (long long)n_out, (long long)c.n_out);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (history <= kWideMax) {   // the whole row in one workgroup
-    return with_wide_vpl(history, [&](auto vpl) {
+    return with_wide_vpl_fine(history, [&](auto vpl) {
       constexpr int VPL = decltype(vpl)::value;
       reuse_final_wide_kernel<VPL, 2><<<static_cast<unsigned>(rows), kWideNT, 0, st>>>(
           scores, scores_ld, nullptr, nullptr, nullptr, 0, 0, static_cast<int>(c.keep), static_cast<int>(history),
