@@ -170,19 +170,25 @@ def check(rc: int) -> None:
         raise RuntimeError(load().qkv_last_error().decode())
 
 
+_STRIDE_ARRAYS = [ctypes.c_int64 * n for n in range(8)]
+
+
 def strides(*vals: int):
-    arr = (ctypes.c_int64 * len(vals))(*[int(v) for v in vals])
-    return arr
+    """A C array of the strides (torch's own ints, taken without conversion)."""
+    return _STRIDE_ARRAYS[len(vals)](*vals)
 
 
 _SAME_DEVICE = contextlib.nullcontext()
+# torch.cuda.current_device() without its lazy-initialisation check: a CUDA
+# tensor exists wherever this is asked
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def on_device(device: torch.device):
     """torch.cuda.device(device), or a no-op when that device is already
     current (the per-call guard costs more than the launch it guards)."""
     idx = device.index
-    if idx is None or torch.cuda.current_device() == idx:
+    if idx is None or _current_device() == idx:
         return _SAME_DEVICE
     return torch.cuda.device(device)
 
