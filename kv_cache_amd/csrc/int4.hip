@@ -440,7 +440,9 @@ int launch_scores(int S, dim3 grid, hipStream_t st, const uint16_t* q, int hq, i
 // Decode scoring of qkv_int4_decode_topk: token scores (block 1), one
 // workgroup per 4096-key chunk of the long-row top-k, each key also counted
 // in the chunk's 12-bit histogram in LDS, and the chunk's top-k window
-// (chunk_window) written where qkv_topk_ws's histogram pass would write it.
+// (chunk_window) written where qkv_topk_ws's histogram pass would write it --
+// or, for a k past the chunk lists, the chunk's counts added to its row's
+// histogram (row_hist).
 // win_waves: the chunk's waves, every wave stage one whole slab tile.
 constexpr int win_waves(int s) {
   return kStageChunk / slab_tile_keys(s) >= 16 ? 16 : static_cast<int>(kStageChunk / slab_tile_keys(s));
@@ -451,7 +453,8 @@ __global__ __launch_bounds__(64 * win_waves(S)) void decode_scores_win_kernel(
     const uint16_t* __restrict__ query, int q_heads, int kv_heads, int head_dim,
     const int32_t* __restrict__ chan_idx, const uint8_t* __restrict__ slab,
     const uint16_t* __restrict__ slab_scales, int64_t capacity, int tokens, int k, float* __restrict__ scores,
-    int n_chunks, int32_t* __restrict__ win, float* __restrict__ qscale_out) {
+    int n_chunks, int32_t* __restrict__ win, int* __restrict__ row_hist, int64_t hist_stride,
+    float* __restrict__ qscale_out) {
   constexpr int NWV = win_waves(S), NT = 64 * NWV;
   static_assert(kStageChunk % (NWV * slab_tile_keys(S)) == 0, "a chunk is whole workgroup stages");
   __shared__ uint32_t h[kHistBins];
@@ -465,6 +468,10 @@ __global__ __launch_bounds__(64 * win_waves(S)) void decode_scores_win_kernel(
                                   1, kStageChunk, scores, tokens, nullptr, nullptr, qscale_out, blockIdx.y,
                                   blockIdx.x, h);
   __syncthreads();
+  if (row_hist) {   // uniform: the row histogram of a large k instead
+    flush_row_hist<NT>(h, row_hist + blockIdx.y * hist_stride);
+    return;
+  }
   const int len = min(kStageChunk, tokens - static_cast<int>(blockIdx.x) * kStageChunk);
   chunk_window<NT, false>(h, min(k, len), win + (static_cast<int64_t>(blockIdx.y) * n_chunks + blockIdx.x) * kWinWords,
                           wsum, &t_sh);
@@ -761,6 +768,11 @@ namespace qkv {
 int topk_filtered(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
                   void* workspace, hipStream_t st, bool given);
 bool topk_takes_windows(int64_t n, int64_t k);
+bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes);
+int64_t topk_least_bytes(int64_t rows, int64_t n, int64_t k);
+int topk_big_clear(int64_t rows, int64_t n, void* workspace, hipStream_t st, int** hist, int64_t* stride);
+int topk_big_finish(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
+                    void* workspace, hipStream_t st);
 }  // namespace qkv
 
 QKV_EXPORT int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_heads, int64_t kv_heads,
@@ -782,12 +794,13 @@ QKV_EXPORT int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_
     return fail(QKV_ERR_INVALID, "%s: capacity must be a multiple of %lld for %lld channels", what,
                 (long long)slab_tile_keys(static_cast<int>(selected)), (long long)selected);
   const int64_t rows = batch * kv_heads;
-  const int64_t need = qkv_topk_workspace_bytes(rows, tokens, k);
+  const int64_t need = topk_least_bytes(rows, tokens, k);
   if (need < 0 || workspace_bytes < need || (need > 0 && !workspace))
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
   if (need > 0 && !aligned(workspace, 16)) return fail(QKV_ERR_INVALID, "%s: workspace must be 16-byte aligned", what);
-  if (!topk_takes_windows(tokens, k) || rows > 65535) {   // the scores, then qkv_topk_ws as it stands
+  const bool row_hist = topk_takes_row_hist(rows, tokens, k, workspace, workspace_bytes);
+  if (!(topk_takes_windows(tokens, k) || row_hist) || rows > 65535) {   // the scores, then qkv_topk_ws as it stands
     if (int rc = qkv_int4_decode_scores(query, batch, q_heads, kv_heads, head_dim, chan_idx, selected, slab,
                                         slab_scales, capacity, tokens, 1, scores, nullptr, nullptr, nullptr, dtype,
                                         stream))
@@ -799,12 +812,17 @@ QKV_EXPORT int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_
   dim3 grid(static_cast<unsigned>(n_chunks), static_cast<unsigned>(rows));
   const uint16_t* q = static_cast<const uint16_t*>(query);
   int32_t* win = static_cast<int32_t*>(workspace);   // qkv_topk_ws's window region
+  int* hist = nullptr;
+  int64_t hist_stride = 0;
+  if (row_hist)
+    if (int rc = topk_big_clear(rows, tokens, workspace, st, &hist, &hist_stride)) return rc;
   auto launch = [&](auto sc, auto fc) {
     constexpr int SS = decltype(sc)::value;
     constexpr bool FF = decltype(fc)::value;
     decode_scores_win_kernel<SS, FF><<<grid, 64 * win_waves(SS), 0, st>>>(
         q, static_cast<int>(q_heads), static_cast<int>(kv_heads), static_cast<int>(head_dim), chan_idx, slab,
-        slab_scales, capacity, static_cast<int>(tokens), static_cast<int>(k), scores, n_chunks, win, nullptr);
+        slab_scales, capacity, static_cast<int>(tokens), static_cast<int>(k), scores, n_chunks, win, hist,
+        hist_stride, nullptr);
     return check_launch(what);
   };
   auto with_f = [&](auto sc) {
@@ -819,5 +837,6 @@ QKV_EXPORT int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_
     default: return fail(QKV_ERR_UNSUPPORTED, "%s: selected channel count %lld not built", what, (long long)selected);
   }
   if (rc) return rc;
+  if (row_hist) return topk_big_finish(scores, rows, tokens, tokens, k, out, workspace, st);
   return topk_filtered(scores, rows, tokens, tokens, k, out, workspace, st, true);
 }

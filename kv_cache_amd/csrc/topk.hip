@@ -1174,6 +1174,288 @@ __global__ __launch_bounds__(1024) void topk_fused_kernel(const float* __restric
   for (int at = kk + tid; at < k; at += 1024) orow[at] = -1;   // not reached: k keys pass the floor
 }
 
+// ---------------------------------------------------------------------------
+// Long rows with a large k (past the chunk lists): the k-th largest key's
+// leading 12 bits from a histogram of the whole row, then slices of the row.
+// topk_rowhist_kernel (or the decode scoring launch) counts every key's top
+// kHistBits order-preserving bits into the row's 4096 global bins, a workgroup
+// histogram in LDS first, one atomic per non-empty bin.  In
+// topk_slices_kernel slice s of a row (1024 * J keys; slot i of wave w covers
+// the row's position word s * 16 * J + w * J + i) finds the boundary bin from
+// that histogram, writes its words with the keys above the bin set, and lists
+// its keys inside the bin in position order (up to `cap`; their true count
+// goes to state[s]).  The row's last slice to take its ticket resolves the
+// bin (from the list in registers, in memory, or, where a slice's list
+// overflowed, from the row itself), sets the taken positions in an LDS bitset
+// of the row and writes the positions in ascending order.  Slices store
+// coherently and complete their stores before the ticket; the last slice
+// reads coherently.  Histogram, counts and tickets are cleared by a fill
+// kernel before the row is counted (the workspace's contents are irrelevant).
+// Bound by latency: the launches and the last slice's passes.  At 32 rows x
+// 32767 keys with k = 3277 BIG1, at 8 rows x 131071 with k = 6554 BIG2 (one
+// workgroup per row: 62 and 222 us).
+// ---------------------------------------------------------------------------
+constexpr int64_t kBigMax = 192 * 1024;    // positions whose bitset fits beside the selection in 64 KB of LDS
+constexpr int kBigSlices = 64;             // slices per row, one lane of a wave each
+constexpr int kBigState = kBigSlices + 8;  // ints per row: the slices' counts, then the ticket
+constexpr int kBigStride = kHistBins + kBigState;   // ints per row of histogram and state
+
+__global__ __launch_bounds__(256) void topk_clear_kernel(int4* __restrict__ p, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) p[i] = make_int4(0, 0, 0, 0);
+}
+
+// One workgroup per kStageChunk keys of a row.
+__global__ __launch_bounds__(1024) void topk_rowhist_kernel(const float* __restrict__ values, int64_t ld, int n,
+                                                            int* __restrict__ hist) {
+  __shared__ uint32_t h[kHistBins];
+  const int tid = threadIdx.x, base = blockIdx.x * kStageChunk;
+  const float* v = values + static_cast<int64_t>(blockIdx.y) * ld;
+  float x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = v[min(base + tid + 1024 * i, n - 1)];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) h[tid + 1024 * i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (base + tid + 1024 * i < n) atomicAdd(&h[f32_sortable(x[i]) >> (32 - kHistBits)], 1u);
+  __syncthreads();
+  flush_row_hist<1024>(h, hist + static_cast<int64_t>(blockIdx.y) * kBigStride);
+}
+
+// The bin's taken keys (above theta, or equal to it among the first kr in
+// position order) as bits of fw, from up to 1024 * VPL of them read by
+// get(p, u, pos) in position order.  The passes start below the bin's digit
+// in sh.hist[1] (clear: boundary() cleared it).
+template <int VPL, typename Get>
+__device__ void bin_taken(void* raw, int m, int rank, int bin, int n, uint64_t* fw, Get&& get) {
+  using WS = WideSelect<VPL, false>;
+  auto& sh = *static_cast<typename WS::Shared*>(raw);
+  WS ws;
+  int at[VPL];
+#pragma unroll
+  for (int i = 0; i < VPL; ++i) {
+    const int p = WS::pos(i);
+    float v = 0.0f;
+    at[i] = 0;
+    if (p < m) get(p, v, at[i]);
+    ws.set(i, v, p < m);
+  }
+  ws.kr = rank;
+  ws.kk = rank;
+  const uint32_t prefix = static_cast<uint32_t>(bin) << (32 - kHistBits);
+  ws.passes(sh, prefix, ~((1u << (32 - kHistBits)) - 1u), 32 - kHistBits, 1, prefix, false);
+  ws.place_uniform(sh, [&](int, int, int slot) {
+    if (static_cast<unsigned>(at[slot]) < static_cast<unsigned>(n))
+      atomicOr(reinterpret_cast<unsigned long long*>(&fw[at[slot] >> 6]), 1ull << (at[slot] & 63));
+  });
+}
+
+// The same for keys too many for registers, read anew on every pass; keys
+// outside the bin may be among them.
+template <typename Get>
+__device__ void bin_taken_stream(void* raw, int m, int rank, int bin, int n, uint64_t* fw, Get&& get) {
+  using WS = WideSelect<1, false>;
+  auto& sh = *static_cast<typename WS::Shared*>(raw);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t bin_mask = ~((1u << (32 - kHistBits)) - 1u), bin_prefix = static_cast<uint32_t>(bin) << (32 - kHistBits);
+  WS ws;
+  ws.kr = rank;
+  uint32_t prefix = bin_prefix, mask = bin_mask;
+  int remaining = 32 - kHistBits, buf = 0;
+#pragma unroll
+  for (int j = 0; j < WS::NB / 1024; ++j) sh.hist[0][tid + 1024 * j] = 0;
+  __syncthreads();
+  while (remaining > 0) {   // uniform
+    const int shift = remaining > WS::RB ? remaining - WS::RB : 0;
+    const uint32_t dmask = (1u << (remaining - shift)) - 1u;
+    for (int p = tid; p < m; p += 1024) {
+      float v;
+      int at;
+      get(p, v, at);
+      const uint32_t u = f32_sortable(v);
+      if ((u & mask) == prefix) atomicAdd(&sh.hist[buf][(u >> shift) & dmask], 1);
+    }
+    __syncthreads();
+    int b, krl, whole;
+    ws.boundary(sh, sh.hist[buf], sh.hist[buf ^ 1], b, krl, whole);
+    prefix |= static_cast<uint32_t>(b) << shift;
+    mask |= dmask << shift;
+    ws.kr = whole ? 0x7FFFFFFF : krl;
+    remaining = whole ? 0 : shift;
+    buf ^= 1;
+    __syncthreads();   // (the histogram's reads are done before the next pass)
+  }
+  // prefix: theta; equal keys are taken while fewer than kr came before
+  const int kr = ws.kr;
+  int eq_seen = 0;   // equal keys in the earlier rounds (uniform)
+  for (int p0 = 0; p0 < m; p0 += 1024) {   // uniform
+    const int p = p0 + tid;
+    float v = 0.0f;
+    int at = 0;
+    if (p < m) get(p, v, at);
+    const uint32_t u = f32_sortable(v);
+    const bool in = p < m && (u & bin_mask) == bin_prefix;
+    const bool gt = in && u > prefix, eq = in && u == prefix;
+    const uint64_t be = __ballot(eq);
+    if (lane == 0) sh.wave_eq[wave] = __popcll(be);
+    __syncthreads();
+    int before = eq_seen, round = 0;
+#pragma unroll
+    for (int w = 0; w < WS::NW; ++w) {
+      before += w < wave ? sh.wave_eq[w] : 0;
+      round += sh.wave_eq[w];
+    }
+    before += static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(be >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(be), 0)));
+    if ((gt || (eq && before < kr)) && static_cast<unsigned>(at) < static_cast<unsigned>(n))
+      atomicOr(reinterpret_cast<unsigned long long*>(&fw[at >> 6]), 1ull << (at & 63));
+    eq_seen += round;
+    __syncthreads();   // (wave_eq is rewritten next round)
+  }
+}
+
+template <int J>
+__global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restrict__ values, int64_t ld, int n, int k,
+                                                           int slices, int cap, int* __restrict__ hist,
+                                                           float* __restrict__ list_val, int* __restrict__ list_pos,
+                                                           uint64_t* __restrict__ words, int32_t* __restrict__ out) {
+  using WS = WideSelect<1, false>;
+  static_assert(sizeof(typename WS::Shared) == sizeof(typename WideSelect<8, false>::Shared),
+                "one shared layout for every list length");
+  extern __shared__ uint64_t fw[];   // the row's taken positions, one bit each
+  __shared__ typename WS::Shared sh;
+  __shared__ int wave_cnt[16];
+  __shared__ int pre[kBigSlices + 1];
+  __shared__ int last_sh, over_sh;
+  const int row = blockIdx.x / slices, s = blockIdx.x - row * slices;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int* hrow = hist + static_cast<int64_t>(row) * kBigStride;
+  int* state = hist + static_cast<int64_t>(row) * kBigStride + kHistBins;
+  const float* vrow = values + static_cast<int64_t>(row) * ld;
+  // the histogram (4 bins per thread) and the slice's keys, all loads in flight
+  const int4 hv = *reinterpret_cast<const int4*>(hrow + 4 * tid);
+  const int w0 = s * 16 * J + wave * J;   // the wave's first word
+  float v[J];
+#pragma unroll
+  for (int i = 0; i < J; ++i) v[i] = vrow[min(64 * (w0 + i) + lane, n - 1)];
+  *reinterpret_cast<int4*>(sh.hist[0] + 4 * tid) = hv;
+  __syncthreads();
+  WS ws;
+  ws.kr = k;
+  int bin, rank, whole;
+  ws.boundary(sh, sh.hist[0], sh.hist[1], bin, rank, whole);
+  const int n_words = (n + 63) / 64;
+  uint64_t* wrow = words + static_cast<int64_t>(row) * n_words;
+  uint64_t bal[J];
+  int wtot = 0;
+#pragma unroll
+  for (int i = 0; i < J; ++i) {
+    const bool in = 64 * (w0 + i) + lane < n;
+    const uint32_t d = f32_sortable(v[i]) >> (32 - kHistBits);
+    const uint64_t w = __ballot(in && d > static_cast<uint32_t>(bin));
+    if (lane == 0 && w0 + i < n_words)
+      __hip_atomic_store(wrow + w0 + i, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bal[i] = __ballot(in && d == static_cast<uint32_t>(bin));
+    wtot += __popcll(bal[i]);
+  }
+  if (lane == 0) wave_cnt[wave] = wtot;
+  __syncthreads();
+  int at = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    at += w < wave ? wave_cnt[w] : 0;
+    total += wave_cnt[w];
+  }
+  if (tid == 0) st_coherent(state + s, total);
+  if (wtot) {   // uniform per wave
+    const int64_t base = (static_cast<int64_t>(row) * slices + s) * cap;
+#pragma unroll
+    for (int i = 0; i < J; ++i) {
+      if ((bal[i] >> lane) & 1ull) {
+        const int e = at + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                               static_cast<uint32_t>(bal[i] >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bal[i]), 0)));
+        if (e < cap) {
+          st_coherent(list_val + base + e, v[i]);
+          st_coherent(list_pos + base + e, 64 * (w0 + i) + lane);
+        }
+      }
+      at += __popcll(bal[i]);
+    }
+  }
+  // Every word, count and list store of this workgroup has completed before its ticket.
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (tid == 0) {
+    // compiler-only fences keep memory operations on their side of the ticket
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const int t = __hip_atomic_fetch_add(state + kBigSlices, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    last_sh = t == slices - 1;
+  }
+  __syncthreads();
+  if (!last_sh) return;
+  // The row's last slice: every slice has stored its words and list.
+  if (tid < 64) {
+    const int c = tid < slices ? ld_coherent(state + tid) : 0;
+    const uint64_t over = __ballot(c > cap);
+    const int inc = wave_incl_scan_dpp(min(c, cap));
+    if (tid < slices) pre[tid + 1] = inc;
+    if (tid == 0) {
+      pre[0] = 0;
+      over_sh = over != 0;
+    }
+  }
+  for (int j = tid; j < n_words; j += 1024)
+    fw[j] = __hip_atomic_load(wrow + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const int64_t lbase = static_cast<int64_t>(row) * slices * cap;
+  auto from_list = [&](int p, float& x, int& pos) {
+    int lo = 0, hi = slices - 1;   // the last slice whose entries start at or before p
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (pre[mid] <= p) lo = mid;
+      else hi = mid - 1;
+    }
+    const int64_t e = lbase + static_cast<int64_t>(lo) * cap + (p - pre[lo]);
+    x = ld_coherent(list_val + e);
+    pos = ld_coherent(list_pos + e);
+  };
+  const int m = pre[slices];
+  if (over_sh)   // uniform
+    bin_taken_stream(&sh, n, rank, bin, n, fw, [&](int p, float& x, int& pos) {
+      x = vrow[p];
+      pos = p;
+    });
+  else if (m <= 1024) bin_taken<1>(&sh, m, rank, bin, n, fw, from_list);
+  else if (m <= 8 * 1024) bin_taken<8>(&sh, m, rank, bin, n, fw, from_list);
+  else bin_taken_stream(&sh, m, rank, bin, n, fw, from_list);
+  __syncthreads();
+  // the taken positions, ascending: consecutive words per thread
+  const int wpt = (n_words + 1023) / 1024;
+  int cnt = 0;
+  for (int j = 0; j < wpt; ++j) {
+    const int w = tid * wpt + j;
+    if (w < n_words) cnt += __popcll(fw[w]);
+  }
+  const int incl = wave_incl_scan_dpp(cnt);
+  if (lane == 63) wave_cnt[wave] = incl;
+  __syncthreads();
+  int p = incl - cnt;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) p += w < wave ? wave_cnt[w] : 0;
+  int32_t* orow = out + static_cast<int64_t>(row) * k;
+  for (int j = 0; j < wpt; ++j) {
+    const int w = tid * wpt + j;
+    if (w >= n_words) break;
+    for (uint64_t x = fw[w]; x; x &= x - 1) {
+      if (p < k) orow[p] = 64 * w + __builtin_ctzll(x);
+      ++p;
+    }
+  }
+}
+
 // Candidates left after a stage over n keys: k from every full chunk, and
 // min(k, rest) from the last.
 int64_t stage_out(int64_t n, int64_t k) {
@@ -1187,6 +1469,47 @@ bool staged(int64_t n, int64_t k) { return n > kStageChunk && k <= kStageMaxK; }
 bool filtered(int64_t n, int64_t k) {
   const int64_t chunks = cdiv(n, kStageChunk);
   return staged(n, k) && chunks <= kFilterMaxChunks && chunks * k <= kFilterMaxLists;
+}
+
+// Rows that take the row histogram and slices: past the chunk lists.
+bool big(int64_t n, int64_t k) { return n > kStageChunk && n <= kBigMax && !filtered(n, k); }
+
+// Keys per thread of a slice: the fewest that keep the grid within 256
+// workgroups (one per CU) and a row within kBigSlices slices.
+int big_j(int64_t rows, int64_t n) {
+  int j = 4;
+  while (j < 32 && (rows * cdiv(n, int64_t(1024) * j) > 256 || cdiv(n, int64_t(1024) * j) > kBigSlices)) j *= 2;
+  return j;
+}
+
+// List entries a slice of 1024 * j keys may hold (a 12-bit bin of normal
+// scores holds some 2% of the keys).
+int64_t big_cap(int j) { return 1024 * j / 8; }
+
+struct BigWs {
+  int* hist;
+  float* list_val;
+  int* list_pos;
+  uint64_t* words;
+  int64_t bytes;
+};
+BigWs big_ws(void* ws, int64_t rows, int64_t n) {
+  const int j = big_j(rows, n);
+  const int64_t entries = rows * cdiv(n, int64_t(1024) * j) * big_cap(j);
+  auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
+  char* p = static_cast<char*>(ws);
+  BigWs w;
+  int64_t at = 0;
+  w.hist = reinterpret_cast<int*>(p + at);
+  at += up(rows * kBigStride * 4);
+  w.list_val = reinterpret_cast<float*>(p + at);
+  at += up(entries * 4);
+  w.list_pos = reinterpret_cast<int*>(p + at);
+  at += up(entries * 4);
+  w.words = reinterpret_cast<uint64_t*>(p + at);
+  at += up(rows * cdiv(n, 64) * 8);
+  w.bytes = at;
+  return w;
 }
 
 template <bool FINITE>
@@ -1318,6 +1641,39 @@ int topk_filtered(const float* values, int64_t rows, int64_t n, int64_t ld, int6
   return check_launch("qkv_topk_ws");
 }
 
+// The row-histogram path (big(n, k)) in its three launches: the clearing,
+// the counting (here, or by a scoring launch that adds to the histogram
+// returned with its row stride) and the slices.
+int topk_big_clear(int64_t rows, int64_t n, void* workspace, hipStream_t st, int** hist, int64_t* stride) {
+  const BigWs w = big_ws(workspace, rows, n);
+  static_assert(kBigStride % 4 == 0, "cleared 16 bytes at a time");
+  const int64_t n4 = rows * kBigStride / 4;
+  topk_clear_kernel<<<static_cast<unsigned>(cdiv(n4, 256)), 256, 0, st>>>(reinterpret_cast<int4*>(w.hist), n4);
+  *hist = w.hist;
+  *stride = kBigStride;
+  return check_launch("qkv_topk_ws");
+}
+
+int topk_big_finish(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
+                    void* workspace, hipStream_t st) {
+  const BigWs w = big_ws(workspace, rows, n);
+  const size_t lds = static_cast<size_t>(cdiv(n, 64)) * 8;
+  auto launch = [&](auto jc) {
+    constexpr int J = decltype(jc)::value;
+    const int64_t slices = cdiv(n, int64_t(1024) * J);
+    topk_slices_kernel<J><<<static_cast<unsigned>(rows * slices), 1024, lds, st>>>(
+        values, ld, static_cast<int>(n), static_cast<int>(k), static_cast<int>(slices), static_cast<int>(big_cap(J)),
+        w.hist, w.list_val, w.list_pos, w.words, out);
+    return check_launch("qkv_topk_ws");
+  };
+  switch (big_j(rows, n)) {
+    case 4: return launch(std::integral_constant<int, 4>{});
+    case 8: return launch(std::integral_constant<int, 8>{});
+    case 16: return launch(std::integral_constant<int, 16>{});
+    default: return launch(std::integral_constant<int, 32>{});
+  }
+}
+
 // Whether qkv_topk_ws takes the histogram-and-filter path for (n, k).
 bool topk_takes_windows(int64_t n, int64_t k) { return filtered(n, k); }
 
@@ -1347,8 +1703,10 @@ QKV_EXPORT int qkv_topk(const float* values, int64_t rows, int64_t n, int64_t ld
   return check_launch("qkv_topk");
 }
 
-QKV_EXPORT int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
-  if (rows <= 0 || n <= 0 || k < 1 || k > n) return -1;
+namespace qkv {
+// Workspace of the paths before the row histogram: none where one workgroup
+// per row selects.  Calls that bring only this much still take those paths.
+static int64_t staged_bytes(int64_t rows, int64_t n, int64_t k) {
   if (!staged(n, k)) return 0;
   const int64_t chunks = cdiv(n, kStageChunk);
   if (filtered(n, k))   // chunk windows, then per-chunk lists of k (value, index) and their counts
@@ -1359,19 +1717,45 @@ QKV_EXPORT int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k) 
          rows * chunks * static_cast<int64_t>(sizeof(uint32_t));
 }
 
+int64_t topk_least_bytes(int64_t rows, int64_t n, int64_t k) {
+  return rows <= 0 || n <= 0 || k < 1 || k > n ? -1 : staged_bytes(rows, n, k);
+}
+
+// Whether a call takes the row-histogram path: its sizes, and a workspace that holds it.
+bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes) {
+  return rows > 0 && rows <= 65535 && k >= 1 && k <= n && big(n, k) && workspace && aligned(workspace, 16) &&
+         bytes >= big_ws(nullptr, rows, n).bytes;
+}
+}  // namespace qkv
+
+QKV_EXPORT int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
+  if (rows <= 0 || n <= 0 || k < 1 || k > n) return -1;
+  return std::max(staged_bytes(rows, n, k), big(n, k) && rows <= 65535 ? big_ws(nullptr, rows, n).bytes : int64_t{0});
+}
+
 QKV_EXPORT int qkv_topk_ws(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
                            void* workspace, int64_t workspace_bytes, void* stream) {
-  if (!staged(n, k)) return qkv_topk(values, rows, n, ld, k, out, stream);
+  const bool row_hist = topk_takes_row_hist(rows, n, k, workspace, workspace_bytes);
+  if (!staged(n, k) && !row_hist) return qkv_topk(values, rows, n, ld, k, out, stream);
   if (!values || !out || !workspace) return fail(QKV_ERR_INVALID, "qkv_topk_ws: null pointer");
   if (rows <= 0 || rows > 65535 || ld < n || n >= (int64_t(1) << 31))
     return fail(QKV_ERR_INVALID, "qkv_topk_ws: bad sizes rows=%lld n=%lld ld=%lld", (long long)rows,
                 (long long)n, (long long)ld);
-  const int64_t need = qkv_topk_workspace_bytes(rows, n, k);
+  const int64_t need = staged_bytes(rows, n, k);
   if (workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "qkv_topk_ws: workspace needs %lld bytes, got %lld", (long long)need,
                 (long long)workspace_bytes);
   if (!aligned(workspace, 16)) return fail(QKV_ERR_INVALID, "qkv_topk_ws: workspace must be 16-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (row_hist) {
+    int* hist;
+    int64_t stride;
+    if (int rc = topk_big_clear(rows, n, workspace, st, &hist, &stride)) return rc;
+    dim3 grid(static_cast<unsigned>(cdiv(n, kStageChunk)), static_cast<unsigned>(rows));
+    topk_rowhist_kernel<<<grid, 1024, 0, st>>>(values, ld, static_cast<int>(n), hist);
+    if (int rc = check_launch("qkv_topk_ws")) return rc;
+    return topk_big_finish(values, rows, n, ld, k, out, workspace, st);
+  }
   const int64_t n1 = stage_out(n, k);
   float* val_buf[2];
   int32_t* idx_buf[2];

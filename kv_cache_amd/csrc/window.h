@@ -83,5 +83,17 @@ __device__ void chunk_window(const uint32_t* h, int target, int32_t* __restrict_
   }
 }
 
+// Adds a workgroup's complete 4096-bin LDS histogram to a row's global one:
+// one device-scope atomic per non-empty bin.  Every thread of NT calls it
+// after the barrier that completed h.
+template <int NT>
+__device__ __forceinline__ void flush_row_hist(const uint32_t* h, int* __restrict__ row_hist) {
+#pragma unroll
+  for (int i = 0; i < kHistBins / NT; ++i) {
+    const int c = static_cast<int>(h[threadIdx.x + NT * i]);
+    if (c) __hip_atomic_fetch_add(row_hist + threadIdx.x + NT * i, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
 }  // namespace
 }  // namespace qkv

@@ -1,0 +1,87 @@
+"""Top-k with k past the chunk lists on long rows (row histogram and slices): every tie pattern, list
+lengths in registers, in memory and overflowing, and the decode call that counts as it scores."""
+
+import numpy as np
+import pytest
+import torch
+
+from kv_cache_amd import _lib
+from kv_cache_amd import int4 as K
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def rows_of(n, seed):
+    g = torch.Generator().manual_seed(seed)
+    few = torch.randint(-3, 4, (n,), generator=g).float()
+    inf = torch.randn(n, generator=g)
+    inf[torch.rand(n, generator=g) < 0.4] = -float("inf")
+    return torch.stack([
+        torch.randn(n, generator=g),                  # some 2% of the keys in the boundary bin
+        few,                                          # large groups of equal keys
+        torch.zeros(n),                               # every key equal: the lists overflow
+        100.0 + torch.rand(n, generator=g),           # one bin: the lists overflow
+        100.0 + 40.0 * torch.rand(n, generator=g),    # a tenth of the keys in a bin
+        inf,
+    ])
+
+
+def want(vals, k):
+    order = np.argsort(-vals.numpy(), axis=1, kind="stable")[:, :k]
+    return np.sort(order, axis=1)
+
+
+@pytest.mark.parametrize("n", [4097, 8192, 20003, 65536, 131072, 196608])
+@pytest.mark.parametrize("share", [0.0, 0.1, 0.5, 1.0])
+@pytest.mark.parametrize("copies", [1, 20])   # 6 or 120 rows: other keys per thread
+def test_large_k_equals_stable_sort(n, share, copies):
+    if copies > 1 and n > 65536:
+        pytest.skip("the same slices as the shorter rows")
+    k = max(1025, min(n, int(share * n)))
+    vals = rows_of(n, n + copies)
+    assert _lib.load().qkv_topk_workspace_bytes(6, n, k) > 0
+    ws = K.topk_workspace(6 * copies, n, k, DEV)
+    ws.fill_(float("nan"))   # contents irrelevant
+    dev = vals.repeat(copies, 1).to(DEV)
+    for _ in range(2):
+        got = K.block_topk(dev, k, workspace=ws).cpu().numpy().reshape(copies, 6, k)
+        assert np.array_equal(got[0], want(vals, k))
+        assert (got == got[:1]).all()
+
+
+def test_calls_without_the_larger_workspace_still_run():
+    lib = _lib.load()
+    vals = rows_of(9000, 4).to(DEV)
+    out = torch.empty((6, 2000), dtype=torch.int32, device=DEV)
+    _lib.check(lib.qkv_topk_ws(vals.data_ptr(), 6, 9000, 9000, 2000, out.data_ptr(), None, 0, _lib.stream_of(vals)))
+    assert np.array_equal(out.cpu().numpy(), want(vals.cpu(), 2000))
+
+
+@pytest.mark.parametrize("tokens,k,selected", [(5000, 1200, 16), (20011, 2002, 32), (70001, 7001, 64), (8192, 8192, 128)])
+def test_decode_topk_counts_as_it_scores(tokens, k, selected):
+    g = torch.Generator().manual_seed(tokens)
+    key = torch.randn((2, 3, tokens, 128), generator=g).to(torch.bfloat16).to(DEV)
+    q = torch.randn((2, 12, 128), generator=g).to(torch.bfloat16).to(DEV)
+    cache = K.Int4KCache.from_prefill(key, 32, selected)
+    scores = torch.empty((2, 3, tokens), device=DEV)
+    got = K.decode_topk(q, cache.chan_idx, cache.slab, cache.slab_scales, tokens, k, scores=scores)
+    bmax = K.decode_scores(q, cache.chan_idx, cache.slab, cache.slab_scales, tokens, 1)
+    assert torch.equal(scores, bmax)
+    assert np.array_equal(got.cpu().numpy().reshape(6, k), want(bmax.cpu().view(6, tokens), k))
+
+
+def test_large_k_in_a_graph():
+    vals = rows_of(30000, 8).to(DEV)
+    ws = K.topk_workspace(6, 30000, 3000, DEV)
+    out = torch.empty((6, 3000), dtype=torch.int32, device=DEV)
+    K.block_topk(vals, 3000, out=out, workspace=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        K.block_topk(vals, 3000, out=out, workspace=ws)
+    for seed in range(3):
+        vals.copy_(rows_of(30000, 50 + seed))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), want(vals.cpu(), 3000))
