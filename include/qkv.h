@@ -247,6 +247,18 @@ int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_heads, int6
                          const uint16_t* slab_scales, int64_t capacity, int64_t tokens, int64_t k, float* scores,
                          int32_t* out, void* workspace, int64_t workspace_bytes, int dtype, void* stream);
 
+/* The same with a state the caller keeps (optional; qkv_topk_state_bytes(rows,
+ * tokens, k) bytes, 16-byte aligned, 0 where the sizes use none): zero-filled
+ * once, left zero by every completed call, so that no launch clears the row
+ * histograms.  Calls sharing a state must not overlap in time and must have
+ * the same number of rows. */
+int64_t qkv_topk_state_bytes(int64_t rows, int64_t n, int64_t k);
+int qkv_int4_decode_topk_state(const void* query, int64_t batch, int64_t q_heads, int64_t kv_heads,
+                               int64_t head_dim, const int32_t* chan_idx, int64_t selected, const uint8_t* slab,
+                               const uint16_t* slab_scales, int64_t capacity, int64_t tokens, int64_t k,
+                               float* scores, int32_t* out, void* workspace, int64_t workspace_bytes,
+                               void* state, int64_t state_bytes, int dtype, void* stream);
+
 /* No counterpart in the reference; for tests of qkv_topk_ws's one-launch
  * path.  Sets how long (ticks of the 100 MHz real-time clock) a chunk waits
  * for the other chunks of its row before keeping its exact top-k instead of

@@ -126,6 +126,9 @@ _PROTOTYPES = {
                                    _i32, _i32, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp]),
     "qkv_int4_decode_topk": (_i32, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _vp, _vp,
                                     _vp, _i64, _i32, _vp]),
+    "qkv_topk_state_bytes": (_i64, [_i64, _i64, _i64]),
+    "qkv_int4_decode_topk_state": (_i32, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _vp,
+                                          _vp, _vp, _i64, _vp, _i64, _i32, _vp]),
     "qkv_reuse_candidates": (_i32, [_vp, _vp, _P(_i64), _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _i64,
                                     _vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp]),
     "qkv_reuse_select_bits": (_i32, [_vp, _vp, _P(_i64), _i32, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i64,

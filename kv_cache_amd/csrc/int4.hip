@@ -770,9 +770,10 @@ int topk_filtered(const float* values, int64_t rows, int64_t n, int64_t ld, int6
 bool topk_takes_windows(int64_t n, int64_t k);
 bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes);
 int64_t topk_least_bytes(int64_t rows, int64_t n, int64_t k);
+int64_t topk_hist_stride();
 int topk_big_clear(int64_t rows, int64_t n, void* workspace, hipStream_t st, int** hist, int64_t* stride);
 int topk_big_finish(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
-                    void* workspace, hipStream_t st);
+                    void* workspace, int* state, hipStream_t st);
 }  // namespace qkv
 
 QKV_EXPORT int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_heads, int64_t kv_heads,
@@ -780,6 +781,17 @@ QKV_EXPORT int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_
                                     const uint8_t* slab, const uint16_t* slab_scales, int64_t capacity,
                                     int64_t tokens, int64_t k, float* scores, int32_t* out, void* workspace,
                                     int64_t workspace_bytes, int dtype, void* stream) {
+  return qkv_int4_decode_topk_state(query, batch, q_heads, kv_heads, head_dim, chan_idx, selected, slab, slab_scales,
+                                    capacity, tokens, k, scores, out, workspace, workspace_bytes, nullptr, 0, dtype,
+                                    stream);
+}
+
+QKV_EXPORT int qkv_int4_decode_topk_state(const void* query, int64_t batch, int64_t q_heads, int64_t kv_heads,
+                                          int64_t head_dim, const int32_t* chan_idx, int64_t selected,
+                                          const uint8_t* slab, const uint16_t* slab_scales, int64_t capacity,
+                                          int64_t tokens, int64_t k, float* scores, int32_t* out, void* workspace,
+                                          int64_t workspace_bytes, void* state, int64_t state_bytes, int dtype,
+                                          void* stream) {
   static const char* what = "qkv_int4_decode_topk";
   if (int rc = check_query(query, batch, q_heads, kv_heads, head_dim, chan_idx, selected, what)) return rc;
   bool f16;
@@ -814,8 +826,19 @@ QKV_EXPORT int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_
   int32_t* win = static_cast<int32_t*>(workspace);   // qkv_topk_ws's window region
   int* hist = nullptr;
   int64_t hist_stride = 0;
-  if (row_hist)
-    if (int rc = topk_big_clear(rows, tokens, workspace, st, &hist, &hist_stride)) return rc;
+  const bool kept = row_hist && state;   // a zero-filled state the caller keeps: nothing to clear
+  if (row_hist) {
+    if (kept) {
+      const int64_t need_state = qkv_topk_state_bytes(rows, tokens, k);
+      if (state_bytes < need_state || !aligned(state, 16))
+        return fail(QKV_ERR_INVALID, "%s: the state needs %lld bytes (16-byte aligned), got %lld", what,
+                    (long long)need_state, (long long)state_bytes);
+      hist = static_cast<int*>(state);
+      hist_stride = topk_hist_stride();
+    } else if (int rc = topk_big_clear(rows, tokens, workspace, st, &hist, &hist_stride)) {
+      return rc;
+    }
+  }
   auto launch = [&](auto sc, auto fc) {
     constexpr int SS = decltype(sc)::value;
     constexpr bool FF = decltype(fc)::value;
@@ -837,6 +860,7 @@ QKV_EXPORT int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_
     default: return fail(QKV_ERR_UNSUPPORTED, "%s: selected channel count %lld not built", what, (long long)selected);
   }
   if (rc) return rc;
-  if (row_hist) return topk_big_finish(scores, rows, tokens, tokens, k, out, workspace, st);
+  if (row_hist)
+    return topk_big_finish(scores, rows, tokens, tokens, k, out, workspace, kept ? hist : nullptr, st);
   return topk_filtered(scores, rows, tokens, tokens, k, out, workspace, st, true);
 }

@@ -1175,8 +1175,8 @@ __global__ __launch_bounds__(1024) void topk_fused_kernel(const float* __restric
 }
 
 // ---------------------------------------------------------------------------
-// Long rows with a large k (past the chunk lists): the k-th largest key's
-// leading 12 bits from a histogram of the whole row, then slices of the row.
+// Long rows: the k-th largest key's leading 12 bits from a histogram of the
+// whole row, then slices of the row.
 // topk_rowhist_kernel (or the decode scoring launch) counts every key's top
 // kHistBits order-preserving bits into the row's 4096 global bins, a workgroup
 // histogram in LDS first, one atomic per non-empty bin.  In
@@ -1189,11 +1189,13 @@ __global__ __launch_bounds__(1024) void topk_fused_kernel(const float* __restric
 // overflowed, from the row itself), sets the taken positions in an LDS bitset
 // of the row and writes the positions in ascending order.  Slices store
 // coherently and complete their stores before the ticket; the last slice
-// reads coherently.  Histogram, counts and tickets are cleared by a fill
-// kernel before the row is counted (the workspace's contents are irrelevant).
-// Bound by latency: the launches and the last slice's passes.  At 32 rows x
-// 32767 keys with k = 3277 BIG1, at 8 rows x 131071 with k = 6554 BIG2 (one
-// workgroup per row: 62 and 222 us).
+// reads coherently.  Histogram, counts and ticket are zero when the row is
+// counted: a fill kernel clears the workspace's (whose contents are
+// irrelevant), a state the caller keeps is put back to zero by the last slice.
+// Bound by latency (the launch, the histogram and keys, the ticket, the last
+// slice's two passes and its output): 11.6 us at 32 rows x 20010 keys with k =
+// 1001 (13.7 in topk_fused_kernel), 12.2 at 8 rows x 131072 with k = 1024
+// (17.4) and at 8 x 131071 with k = 6554 (222 us, one workgroup per row).
 // ---------------------------------------------------------------------------
 constexpr int64_t kBigMax = 192 * 1024;    // positions whose bitset fits beside the selection in 64 KB of LDS
 constexpr int kBigSlices = 64;             // slices per row, one lane of a wave each
@@ -1320,7 +1322,7 @@ template <int J>
 __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restrict__ values, int64_t ld, int n, int k,
                                                            int slices, int cap, int* __restrict__ hist,
                                                            float* __restrict__ list_val, int* __restrict__ list_pos,
-                                                           uint64_t* __restrict__ words, int32_t* __restrict__ out) {
+                                                           uint64_t* __restrict__ words, int32_t* __restrict__ out, int reset) {
   using WS = WideSelect<1, false>;
   static_assert(sizeof(typename WS::Shared) == sizeof(typename WideSelect<8, false>::Shared),
                 "one shared layout for every list length");
@@ -1412,23 +1414,30 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
   __syncthreads();
   const int64_t lbase = static_cast<int64_t>(row) * slices * cap;
   auto from_list = [&](int p, float& x, int& pos) {
-    int lo = 0, hi = slices - 1;   // the last slice whose entries start at or before p
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (pre[mid] <= p) lo = mid;
-      else hi = mid - 1;
+    int lo = 0;   // the last slice whose entries start at or before p, in fixed steps
+#pragma unroll
+    for (int step = kBigSlices / 2; step > 0; step >>= 1) {
+      const int mid = lo + step;
+      lo = (mid < slices && pre[min(mid, slices)] <= p) ? mid : lo;
     }
     const int64_t e = lbase + static_cast<int64_t>(lo) * cap + (p - pre[lo]);
     x = ld_coherent(list_val + e);
     pos = ld_coherent(list_pos + e);
   };
   const int m = pre[slices];
+  // (every slice has read the histogram: with `reset` it goes back to zero for the next call)
+  if (reset) {
+    *reinterpret_cast<int4*>(hist + static_cast<int64_t>(row) * kBigStride + 4 * tid) = make_int4(0, 0, 0, 0);
+    if (tid < kBigState) state[tid] = 0;
+  }
   if (over_sh)   // uniform
     bin_taken_stream(&sh, n, rank, bin, n, fw, [&](int p, float& x, int& pos) {
       x = vrow[p];
       pos = p;
     });
   else if (m <= 1024) bin_taken<1>(&sh, m, rank, bin, n, fw, from_list);
+  else if (m <= 2 * 1024) bin_taken<2>(&sh, m, rank, bin, n, fw, from_list);
+  else if (m <= 4 * 1024) bin_taken<4>(&sh, m, rank, bin, n, fw, from_list);
   else if (m <= 8 * 1024) bin_taken<8>(&sh, m, rank, bin, n, fw, from_list);
   else bin_taken_stream(&sh, m, rank, bin, n, fw, from_list);
   __syncthreads();
@@ -1471,8 +1480,15 @@ bool filtered(int64_t n, int64_t k) {
   return staged(n, k) && chunks <= kFilterMaxChunks && chunks * k <= kFilterMaxLists;
 }
 
-// Rows that take the row histogram and slices: past the chunk lists.
-bool big(int64_t n, int64_t k) { return n > kStageChunk && n <= kBigMax && !filtered(n, k); }
+// Rows that take the row histogram and slices: every row longer than the
+// one-workgroup selections take.  Decode steps of a token selection that
+// keeps its state, against the chunk lists (us a layer): 8 rows x 4500 23.6
+// (33.1), 8 x 8000 24.3 (27.0), 64 x 7000 29.9 (32.4), 8 x 131072 32.8
+// (39.3), 256 x 5000 33.0 (33.1); block maxima, which also pay the clearing
+// and the counting launch: 8 rows x 6250 37.1 (45.2), 64 x 8192 73.5 (79.2).
+// The chunk lists stay for rows past kBigMax and for calls whose workspace
+// was sized for them.
+bool big(int64_t n) { return n > kStageChunk && n <= kBigMax; }
 
 // Keys per thread of a slice: the fewest that keep the grid within 256
 // workgroups (one per CU) and a row within kBigSlices slices.
@@ -1641,7 +1657,10 @@ int topk_filtered(const float* values, int64_t rows, int64_t n, int64_t ld, int6
   return check_launch("qkv_topk_ws");
 }
 
-// The row-histogram path (big(n, k)) in its three launches: the clearing,
+// The histogram and state of the row-histogram path, at the start of its workspace.
+int64_t big_state_bytes(int64_t rows) { return (rows * kBigStride * 4 + 255) / 256 * 256; }
+
+// The row-histogram path (big(n)) in its three launches: the clearing,
 // the counting (here, or by a scoring launch that adds to the histogram
 // returned with its row stride) and the slices.
 int topk_big_clear(int64_t rows, int64_t n, void* workspace, hipStream_t st, int** hist, int64_t* stride) {
@@ -1654,16 +1673,19 @@ int topk_big_clear(int64_t rows, int64_t n, void* workspace, hipStream_t st, int
   return check_launch("qkv_topk_ws");
 }
 
+// state: the zero-filled histogram and state to use (and to leave zero)
+// instead of the workspace's, or null.
 int topk_big_finish(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
-                    void* workspace, hipStream_t st) {
-  const BigWs w = big_ws(workspace, rows, n);
+                    void* workspace, int* state, hipStream_t st) {
+  BigWs w = big_ws(workspace, rows, n);
+  if (state) w.hist = state;
   const size_t lds = static_cast<size_t>(cdiv(n, 64)) * 8;
   auto launch = [&](auto jc) {
     constexpr int J = decltype(jc)::value;
     const int64_t slices = cdiv(n, int64_t(1024) * J);
     topk_slices_kernel<J><<<static_cast<unsigned>(rows * slices), 1024, lds, st>>>(
         values, ld, static_cast<int>(n), static_cast<int>(k), static_cast<int>(slices), static_cast<int>(big_cap(J)),
-        w.hist, w.list_val, w.list_pos, w.words, out);
+        w.hist, w.list_val, w.list_pos, w.words, out, state ? 1 : 0);
     return check_launch("qkv_topk_ws");
   };
   switch (big_j(rows, n)) {
@@ -1717,20 +1739,27 @@ static int64_t staged_bytes(int64_t rows, int64_t n, int64_t k) {
          rows * chunks * static_cast<int64_t>(sizeof(uint32_t));
 }
 
+int64_t topk_hist_stride() { return kBigStride; }
+
 int64_t topk_least_bytes(int64_t rows, int64_t n, int64_t k) {
   return rows <= 0 || n <= 0 || k < 1 || k > n ? -1 : staged_bytes(rows, n, k);
 }
 
 // Whether a call takes the row-histogram path: its sizes, and a workspace that holds it.
 bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes) {
-  return rows > 0 && rows <= 65535 && k >= 1 && k <= n && big(n, k) && workspace && aligned(workspace, 16) &&
+  return rows > 0 && rows <= 65535 && k >= 1 && k <= n && big(n) && workspace && aligned(workspace, 16) &&
          bytes >= big_ws(nullptr, rows, n).bytes;
 }
 }  // namespace qkv
 
+QKV_EXPORT int64_t qkv_topk_state_bytes(int64_t rows, int64_t n, int64_t k) {
+  if (rows <= 0 || n <= 0 || k < 1 || k > n) return -1;
+  return big(n) && rows <= 65535 ? big_state_bytes(rows) : 0;
+}
+
 QKV_EXPORT int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
   if (rows <= 0 || n <= 0 || k < 1 || k > n) return -1;
-  return std::max(staged_bytes(rows, n, k), big(n, k) && rows <= 65535 ? big_ws(nullptr, rows, n).bytes : int64_t{0});
+  return std::max(staged_bytes(rows, n, k), big(n) && rows <= 65535 ? big_ws(nullptr, rows, n).bytes : int64_t{0});
 }
 
 QKV_EXPORT int qkv_topk_ws(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
@@ -1754,7 +1783,7 @@ QKV_EXPORT int qkv_topk_ws(const float* values, int64_t rows, int64_t n, int64_t
     dim3 grid(static_cast<unsigned>(cdiv(n, kStageChunk)), static_cast<unsigned>(rows));
     topk_rowhist_kernel<<<grid, 1024, 0, st>>>(values, ld, static_cast<int>(n), hist);
     if (int rc = check_launch("qkv_topk_ws")) return rc;
-    return topk_big_finish(values, rows, n, ld, k, out, workspace, st);
+    return topk_big_finish(values, rows, n, ld, k, out, workspace, nullptr, st);
   }
   const int64_t n1 = stage_out(n, k);
   float* val_buf[2];

@@ -196,12 +196,13 @@ def decode_scores(query: torch.Tensor, chan_idx: torch.Tensor, slab: torch.Tenso
 
 def decode_topk(query: torch.Tensor, chan_idx: torch.Tensor, slab: torch.Tensor, slab_scales: torch.Tensor,
                 tokens: int, k: int, *, scores: torch.Tensor | None = None, out: torch.Tensor | None = None,
-                workspace: torch.Tensor | None = None) -> torch.Tensor:
+                workspace: torch.Tensor | None = None, state: torch.Tensor | None = None) -> torch.Tensor:
     """``decode_scores`` with block 1 then ``block_topk`` in one call
     (qkv_int4_decode_topk): the top-k token indices int32 [B, Hkv, k],
     ascending, lowest index first among equal scores; the token scores go to
     ``scores`` f32 [B, Hkv, tokens].  Long rows build the top-k's chunk
-    histograms while they score."""
+    histograms while they score.  ``state`` (from ``topk_state``) is kept zero
+    from call to call and saves the launch that clears it."""
     lib = _lib.load()
     code = _check_query(query)
     _require(slab.is_cuda and slab.dtype == torch.uint8 and slab.is_contiguous(), "slab must be contiguous CUDA uint8")
@@ -223,11 +224,21 @@ def decode_topk(query: torch.Tensor, chan_idx: torch.Tensor, slab: torch.Tensor,
     if need > 0 and (workspace is None or workspace.numel() * 4 < need):
         workspace = topk_workspace(b * hkv, t, k, q.device)
     with _lib.on_device(q.device):
-        _lib.check(lib.qkv_int4_decode_topk(q.data_ptr(), b, hq, hkv, d, chan_idx.data_ptr(), s, slab.data_ptr(),
-                                            slab_scales.data_ptr(), cap, t, int(k), scores.data_ptr(), out.data_ptr(),
-                                            _lib.ptr(workspace), 0 if workspace is None else workspace.numel() * 4,
-                                            code, _lib.stream_of(q)))
+        _lib.check(lib.qkv_int4_decode_topk_state(
+            q.data_ptr(), b, hq, hkv, d, chan_idx.data_ptr(), s, slab.data_ptr(), slab_scales.data_ptr(), cap, t,
+            int(k), scores.data_ptr(), out.data_ptr(), _lib.ptr(workspace),
+            0 if workspace is None else workspace.numel() * 4, _lib.ptr(state),
+            0 if state is None else state.numel() * 4, code, _lib.stream_of(q)))
     return out
+
+
+def topk_state(rows: int, n: int, k: int, device) -> torch.Tensor | None:
+    """Zero-filled state for ``decode_topk`` calls of these sizes (None where
+    they use none); every completed call leaves it zero.  Calls sharing a
+    state must not overlap in time."""
+    need = _lib.load().qkv_topk_state_bytes(int(rows), int(n), int(k))
+    _require(need >= 0, f"bad top-k sizes rows={rows} n={n} k={k}")
+    return torch.zeros(need // 4, dtype=torch.int32, device=device) if need else None
 
 
 def topk_workspace(rows: int, n: int, k: int, device) -> torch.Tensor | None:
@@ -465,6 +476,7 @@ class SparseDecodeStep:
         self.bmax = torch.empty((batch, kv_heads, nb), dtype=torch.float32, device=device)
         self.sel = torch.empty((batch, kv_heads, topk), dtype=torch.int32, device=device)
         self.topk_ws = topk_workspace(batch * kv_heads, nb, topk, device)
+        self.topk_state = topk_state(batch * kv_heads, nb, topk, device) if block == 1 else None
         n_ws = protected_workspace_blocks(topk, block, self.scored, self.protect_sink, self.protect_recent,
                                           self.keep_self)
         self.workspace = attention_workspace(batch, q_heads, kv_heads, head_dim, n_ws, block, device)
@@ -512,7 +524,7 @@ class SparseDecodeStep:
                                            scaling, workspace=self.workspace, sel_out=self.sel, out=self.out, **prot)
         if self.block == 1:   # token selection: the scoring launch feeds the top-k its chunk histograms
             decode_topk(query, cache.chan_idx, cache.slab, cache.slab_scales, self.scored, self.topk,
-                        scores=self.bmax, out=self.sel, workspace=self.topk_ws)
+                        scores=self.bmax, out=self.sel, workspace=self.topk_ws, state=self.topk_state)
         else:
             decode_scores(query, cache.chan_idx, cache.slab, cache.slab_scales, self.scored, self.block,
                           bmax=self.bmax)

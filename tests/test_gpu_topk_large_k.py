@@ -85,3 +85,34 @@ def test_large_k_in_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(out.cpu().numpy(), want(vals.cpu(), 3000))
+
+
+@pytest.mark.parametrize("tokens,k", [(4097, 1), (9001, 300), (40000, 1024), (131072, 4000)])
+def test_kept_state_returns_to_zero(tokens, k):
+    g = torch.Generator().manual_seed(k)
+    key = torch.randn((1, 4, tokens, 128), generator=g).to(torch.bfloat16).to(DEV)
+    cache = K.Int4KCache.from_prefill(key, 32, 32)
+    state = K.topk_state(4, tokens, k, DEV)
+    ws = K.topk_workspace(4, tokens, k, DEV)
+    for seed in range(3):
+        q = torch.randn((1, 8, 128), generator=g).to(torch.bfloat16).to(DEV)
+        scores = torch.empty((1, 4, tokens), device=DEV)
+        got = K.decode_topk(q, cache.chan_idx, cache.slab, cache.slab_scales, tokens, k, scores=scores, workspace=ws,
+                            state=state)
+        assert np.array_equal(got.cpu().numpy().reshape(4, k), want(scores.cpu().view(4, tokens), k))
+        assert int(state.abs().sum()) == 0
+    with pytest.raises(RuntimeError, match="state needs"):
+        K.decode_topk(q, cache.chan_idx, cache.slab, cache.slab_scales, tokens, k, workspace=ws, state=state[:64])
+
+
+@pytest.mark.parametrize("n,k", [(5000, 64), (9000, 1000), (131072, 1024), (196609, 500)])
+def test_smaller_workspaces_take_the_chunk_lists(n, k):
+    """Workspaces sized for the chunk lists (their size does not depend on the row histogram) are still accepted."""
+    vals = rows_of(n, k).to(DEV)
+    chunks = -(-n // 4096)
+    ws = torch.empty(6 * chunks * (66 + 2 * k + 1), dtype=torch.float32, device=DEV)
+    out = torch.empty((6, k), dtype=torch.int32, device=DEV)
+    lib = _lib.load()
+    _lib.check(lib.qkv_topk_ws(vals.data_ptr(), 6, n, n, k, out.data_ptr(), ws.data_ptr(), ws.numel() * 4,
+                               _lib.stream_of(vals)))
+    assert np.array_equal(out.cpu().numpy(), want(vals.cpu(), k))
