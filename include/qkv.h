@@ -772,6 +772,17 @@ int qkv_block_scan_scores(const void* query, const void* key_dim_major, const in
                           int64_t block, int64_t dim_count, float scaling, float* out, float* full, int64_t out_ld,
                           int dtype, void* stream);
 
+/* The same on the n_scan best of the row's ceil(history / block) block scores
+ * (f32 [rows, bscore_ld], the selection of qkv_topk: lowest index first on
+ * ties, ascending), selected in the launch and written to blocks; at most
+ * 1024 blocks. */
+int qkv_block_select_scan_scores(const void* query, const void* key_dim_major, const int64_t* kdm_strides,
+                                 const void* key, const int64_t* k_strides, int64_t batch, int64_t q_heads,
+                                 int64_t kv_heads, int64_t history, int64_t head_dim, const float* bscore,
+                                 int64_t bscore_ld, int32_t* blocks, int64_t n_scan, int64_t block,
+                                 int64_t dim_count, float scaling, float* out, float* full, int64_t out_ld,
+                                 int dtype, void* stream);
+
 /* Block scores of the qboracle selector (EV:5030-5044): out[r, j] = the
  * largest partial score, on row r's top-|q| dims (ties to the lower dim,
  * summed in selection order), of block j's history tokens

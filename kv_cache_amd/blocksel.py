@@ -32,6 +32,7 @@ from .int4 import block_topk, topk_workspace
 from .reuse import dim_major_append, token_attention
 
 QBB, BREP = 0, 1   # QKV_BLOCK_QBB, QKV_BLOCK_BREP
+SCAN_SELECT_BLOCKS = 1024   # rows of at most this many blocks select inside the scan's launch
 QBORACLE = 2       # block maxima of the partial scores: no per-block metadata
 
 
@@ -212,17 +213,25 @@ class BlockSelectDecodeStep:
                     self.q_heads, self.kv_heads, history, self.head_dim, self.block, self.reps, self.dims,
                     self.bscore.data_ptr(), self.meta_blocks, self.dtype_code, stream))
             blocks = self.blocks[: self.rows * n_scan].view(self.rows, n_scan)
-            block_topk(self.bscore[:, :nb], n_scan, out=blocks, workspace=self.topk_ws)
             n_tok = n_scan * self.block
             partial = self.partial[: self.rows * n_tok]
             # the one-workgroup rerank ranks its candidates by the full scores the
             # scan computes for every scanned token; the general one (ws_need > 0)
             # computes them for its candidates only
             full = self.full[: self.rows * n_tok] if ws_need == 0 else None
-            _lib.check(lib.qkv_block_scan_scores(
-                q.data_ptr(), self.kdm.data_ptr(), _lib.strides(*self.kdm.stride()), key.data_ptr(), ks, self.batch,
-                self.q_heads, self.kv_heads, history, self.head_dim, blocks.data_ptr(), n_scan, self.block,
-                self.dims, float(scaling), partial.data_ptr(), _lib.ptr(full), n_tok, self.dtype_code, stream))
+            if nb <= SCAN_SELECT_BLOCKS:   # the scan's launch selects its blocks
+                _lib.check(lib.qkv_block_select_scan_scores(
+                    q.data_ptr(), self.kdm.data_ptr(), _lib.strides(*self.kdm.stride()), key.data_ptr(), ks,
+                    self.batch, self.q_heads, self.kv_heads, history, self.head_dim, self.bscore.data_ptr(),
+                    self.meta_blocks, blocks.data_ptr(), n_scan, self.block, self.dims, float(scaling),
+                    partial.data_ptr(), _lib.ptr(full), n_tok, self.dtype_code, stream))
+            else:
+                block_topk(self.bscore[:, :nb], n_scan, out=blocks, workspace=self.topk_ws)
+                _lib.check(lib.qkv_block_scan_scores(
+                    q.data_ptr(), self.kdm.data_ptr(), _lib.strides(*self.kdm.stride()), key.data_ptr(), ks,
+                    self.batch, self.q_heads, self.kv_heads, history, self.head_dim, blocks.data_ptr(), n_scan,
+                    self.block, self.dims, float(scaling), partial.data_ptr(), _lib.ptr(full), n_tok,
+                    self.dtype_code, stream))
             n_out = int(lib.qkv_final_list_count(history, n_keep, self.sink, self.recent, int(self.keep_self)))
             ids = self.attn_ids[: self.rows * n_out]
             _lib.check(lib.qkv_block_rerank(

@@ -65,11 +65,7 @@ __device__ __forceinline__ uint16_t half_bits(float v) {
 // q is read eight values per 16-byte word where it is used (the empty asm
 // keeps those reads from being hoisted all at once next to the row loads).
 template <bool F16>
-__device__ __forceinline__ float full_score(const uint16_t* __restrict__ krow, const float* q_s, float scaling) {
-  const uint4* kr = reinterpret_cast<const uint4*>(krow);
-  uint4 x[kHD / 8];
-#pragma unroll
-  for (int c = 0; c < kHD / 8; ++c) x[c] = kr[c];
+__device__ __forceinline__ float full_sum(const uint4 (&x)[kHD / 8], const float* q_s, float scaling) {
   const float4* q4 = reinterpret_cast<const float4*>(q_s);
   float acc = 0.0f;
 #pragma unroll
@@ -85,6 +81,14 @@ __device__ __forceinline__ float full_score(const uint16_t* __restrict__ krow, c
     }
   }
   return acc * scaling;
+}
+template <bool F16>
+__device__ __forceinline__ float full_score(const uint16_t* __restrict__ krow, const float* q_s, float scaling) {
+  const uint4* kr = reinterpret_cast<const uint4*>(krow);
+  uint4 x[kHD / 8];
+#pragma unroll
+  for (int c = 0; c < kHD / 8; ++c) x[c] = kr[c];
+  return full_sum<F16>(x, q_s, scaling);
 }
 
 // ---------------------------------------------------------------------------
@@ -289,26 +293,51 @@ __global__ __launch_bounds__(kBT) void block_scores_kernel(
 // dim-major copy: position p of a row is token blocks[p / block] * block +
 // p % block; positions at or past the history score -inf.
 // ---------------------------------------------------------------------------
-template <bool F16>
+// SELV > 0: the blocks are not given; every workgroup of a row selects the
+// n_scan best of the row's nb block scores into LDS (the selection of
+// qkv_topk, SELV keys per thread, repeated by the row's few workgroups instead
+// of launched) and the first writes them to `blocks`.  The token's whole K row
+// (for `full`) and its values on the selected dims are all in flight before
+// either is summed.  32 rows, 513 blocks of 64, 16 scanned, with the
+// selection: 10.9 us (4.2 + 9.0 us as two launches with the row loads behind
+// the partial score).
+template <bool F16, int SELV>
 __global__ __launch_bounds__(kBT) void scan_partial_kernel(
     const uint16_t* __restrict__ query, const uint16_t* __restrict__ kdm, int q_heads, int group, int64_t db,
-    int64_t dh, int64_t dd, const int32_t* __restrict__ blocks, int n_scan, int block, int history, int count,
+    int64_t dh, int64_t dd, int32_t* __restrict__ blocks, int n_scan, int block, int history, int count,
     float* __restrict__ out, int64_t out_ld, const uint16_t* __restrict__ key, int64_t sb, int64_t sh, int64_t st,
-    float scaling, float* __restrict__ full) {
+    float scaling, float* __restrict__ full, const float* __restrict__ bscore, int64_t bscore_ld, int nb) {
   __shared__ __attribute__((aligned(16))) float q_s[kHD];
   __shared__ int sel_idx[kHD];
   __shared__ float sel_q[kHD];
+  __shared__ int32_t sel[SELV > 0 ? kBT * SELV : 1];
   const int row = blockIdx.y, tid = threadIdx.x;
   const int b = row / q_heads, h = row - b * q_heads;
-  for (int d = tid; d < kHD; d += kBT) q_s[d] = half_to_f32<F16>(query[static_cast<int64_t>(row) * kHD + d]);
-  __syncthreads();
-  rank_dims(q_s, count, sel_idx, sel_q);
+  const float q0 = half_to_f32<F16>(query[static_cast<int64_t>(row) * kHD + (tid & (kHD - 1))]);
+  if constexpr (SELV > 0) {
+    select_row<SELV, false, kBT / 64>(bscore + row * bscore_ld, nb, n_scan, sel);
+    if (blockIdx.x == 0)
+      for (int i = tid; i < n_scan; i += kBT) blocks[static_cast<int64_t>(row) * n_scan + i] = sel[i];
+  }
   const int p = blockIdx.x * kBT + tid;
+  const int jb = min(p / block, n_scan - 1);
+  int id;
+  if constexpr (SELV > 0) id = sel[jb];
+  else id = blocks[static_cast<int64_t>(row) * n_scan + jb];
+  const int tok = p < n_scan * block ? id * block + (p - jb * block) : -1;
+  const bool in = tok >= 0 && tok < history;
+  // (positions without a token load the first one's row, unused)
+  uint4 x[kHD / 8];
+  if (full) {   // uniform
+    const uint4* kr = reinterpret_cast<const uint4*>(key + b * sb + (h / group) * sh + static_cast<int64_t>(in ? tok : 0) * st);
+#pragma unroll
+    for (int c = 0; c < kHD / 8; ++c) x[c] = kr[c];
+  }
+  if (tid < kHD) q_s[tid] = q0;
+  rank_dims(q_s, count, sel_idx, sel_q);   // (begins with a barrier)
   if (p >= n_scan * block) return;
-  const int jb = p / block;
-  const int tok = blocks[static_cast<int64_t>(row) * n_scan + jb] * block + (p - jb * block);
   float acc = -__builtin_huge_valf();
-  if (tok >= 0 && tok < history) {
+  if (in) {
     const uint16_t* base = kdm + b * db + (h / group) * dh + tok;
     acc = 0.0f;
     for (int s0 = 0; s0 < count; s0 += 8) {   // eight dims' loads in flight, added in order
@@ -321,12 +350,8 @@ __global__ __launch_bounds__(kBT) void scan_partial_kernel(
     }
   }
   out[static_cast<int64_t>(row) * out_ld + p] = acc;
-  if (full) {   // the full-D score the rerank ranks its candidates by (every scanned position)
-    const bool in = tok >= 0 && tok < history;
-    const float f = in ? full_score<F16>(key + b * sb + (h / group) * sh + static_cast<int64_t>(tok) * st, q_s, scaling)
-                       : -__builtin_huge_valf();
-    full[static_cast<int64_t>(row) * out_ld + p] = f;
-  }
+  if (full)   // the full-D score the rerank ranks its candidates by (every scanned position)
+    full[static_cast<int64_t>(row) * out_ld + p] = in ? full_sum<F16>(x, q_s, scaling) : -__builtin_huge_valf();
 }
 
 // ---------------------------------------------------------------------------
@@ -838,12 +863,18 @@ QKV_EXPORT int qkv_block_scores(int kind, const void* query, const void* key, co
 #undef QKV_BLOCK_SCORES
 }
 
-QKV_EXPORT int qkv_block_scan_scores(const void* query, const void* key_dim_major, const int64_t* kdm_strides,
-                                     const void* key, const int64_t* k_strides, int64_t batch, int64_t q_heads,
-                                     int64_t kv_heads, int64_t history, int64_t head_dim, const int32_t* blocks,
-                                     int64_t n_scan, int64_t block, int64_t dim_count, float scaling, float* out,
-                                     float* full, int64_t out_ld, int dtype, void* stream) {
-  const char* what = "qkv_block_scan_scores";
+// Block scores of at most this many blocks select inside the scan's launch:
+// 32 rows x 513 blocks, 4 workgroups a row, 39.7 -> 38.7 us a layer; 256 rows
+// x 250, 2 a row, 48.4 -> 45.9; past it a row has more workgroups to repeat a
+// longer selection (96 rows x 2063, 16 a row, 88.8 -> 90.2).
+constexpr int64_t kScanSelectBlocks = kBT * 4;
+
+// qkv_block_scan_scores, or with bscore its selecting form.
+static int run_scan(const char* what, const void* query, const void* key_dim_major, const int64_t* kdm_strides,
+                    const void* key, const int64_t* k_strides, int64_t batch, int64_t q_heads, int64_t kv_heads,
+                    int64_t history, int64_t head_dim, int32_t* blocks, int64_t n_scan, int64_t block,
+                    int64_t dim_count, float scaling, float* out, float* full, int64_t out_ld, const float* bscore,
+                    int64_t bscore_ld, int64_t nb, int dtype, void* stream) {
   int rc = check_rows(what, batch, q_heads, kv_heads, head_dim);
   if (rc) return rc;
   bool f16;
@@ -857,15 +888,46 @@ QKV_EXPORT int qkv_block_scan_scores(const void* query, const void* key_dim_majo
     return fail(QKV_ERR_INVALID, "%s: K rows must be contiguous and 16-byte aligned", what);
   const int count = static_cast<int>(std::min<int64_t>(std::max<int64_t>(dim_count, 1), kHD));
   dim3 grid(static_cast<unsigned>(cdiv(n_scan * block, kBT)), static_cast<unsigned>(batch * q_heads));
-  return with_half(f16, [&](auto ff) {
-    scan_partial_kernel<decltype(ff)::value><<<grid, kBT, 0, static_cast<hipStream_t>(stream)>>>(
+  auto launch = [&](auto ff, auto vv) {
+    scan_partial_kernel<decltype(ff)::value, decltype(vv)::value><<<grid, kBT, 0, static_cast<hipStream_t>(stream)>>>(
         static_cast<const uint16_t*>(query), static_cast<const uint16_t*>(key_dim_major), static_cast<int>(q_heads),
         static_cast<int>(q_heads / kv_heads), kdm_strides[0], kdm_strides[1], kdm_strides[2], blocks,
         static_cast<int>(n_scan), static_cast<int>(block), static_cast<int>(history), count, out, out_ld,
         static_cast<const uint16_t*>(key), full ? k_strides[0] : 0, full ? k_strides[1] : 0,
-        full ? k_strides[2] : 0, scaling, full);
+        full ? k_strides[2] : 0, scaling, full, bscore, bscore_ld, static_cast<int>(nb));
     return check_launch(what);
+  };
+  return with_half(f16, [&](auto ff) {
+    if (!bscore) return launch(ff, std::integral_constant<int, 0>{});
+    return launch(ff, std::integral_constant<int, 4>{});
   });
+}
+
+QKV_EXPORT int qkv_block_scan_scores(const void* query, const void* key_dim_major, const int64_t* kdm_strides,
+                                     const void* key, const int64_t* k_strides, int64_t batch, int64_t q_heads,
+                                     int64_t kv_heads, int64_t history, int64_t head_dim, const int32_t* blocks,
+                                     int64_t n_scan, int64_t block, int64_t dim_count, float scaling, float* out,
+                                     float* full, int64_t out_ld, int dtype, void* stream) {
+  return run_scan("qkv_block_scan_scores", query, key_dim_major, kdm_strides, key, k_strides, batch, q_heads, kv_heads,
+                  history, head_dim, const_cast<int32_t*>(blocks), n_scan, block, dim_count, scaling, out, full, out_ld,
+                  nullptr, 0, 0, dtype, stream);
+}
+
+QKV_EXPORT int qkv_block_select_scan_scores(const void* query, const void* key_dim_major, const int64_t* kdm_strides,
+                                            const void* key, const int64_t* k_strides, int64_t batch, int64_t q_heads,
+                                            int64_t kv_heads, int64_t history, int64_t head_dim, const float* bscore,
+                                            int64_t bscore_ld, int32_t* blocks, int64_t n_scan, int64_t block,
+                                            int64_t dim_count, float scaling, float* out, float* full, int64_t out_ld,
+                                            int dtype, void* stream) {
+  const char* what = "qkv_block_select_scan_scores";
+  const int64_t nb = block > 0 && history > 0 ? cdiv(history, block) : 0;
+  if (!bscore || nb < 1 || n_scan > nb || bscore_ld < nb)
+    return fail(QKV_ERR_INVALID, "%s: need block scores of n_scan <= ceil(history / block) <= bscore_ld blocks", what);
+  if (nb > kScanSelectBlocks)
+    return fail(QKV_ERR_UNSUPPORTED, "%s: at most %lld blocks (got %lld); select with qkv_topk_ws first", what,
+                (long long)kScanSelectBlocks, (long long)nb);
+  return run_scan(what, query, key_dim_major, kdm_strides, key, k_strides, batch, q_heads, kv_heads, history, head_dim,
+                  blocks, n_scan, block, dim_count, scaling, out, full, out_ld, bscore, bscore_ld, nb, dtype, stream);
 }
 
 QKV_EXPORT int qkv_block_max_partial_scores(const void* query, const void* key_dim_major, const int64_t* kdm_strides,

@@ -284,3 +284,33 @@ def test_rerank_with_and_without_scan_full_scores(mode, t):
             0, None, 0, 0, _lib.stream_of(q)))
         assert torch.equal(keep[:, :t], want_mask), full is None
         assert torch.equal(ids, want_ids), full is None
+
+
+@pytest.mark.parametrize("nb,n_scan,block", [(1, 1, 16), (256, 7, 4), (257, 257, 4), (1000, 90, 16), (1024, 16, 2)])
+@pytest.mark.parametrize("full", [True, False])
+def test_scan_that_selects_equals_topk_then_scan(nb, n_scan, block, full):
+    lib = _lib.load()
+    b, hkv, hq, t = 2, 2, 4, nb * block - min(block - 1, 1)
+    k, _, g = _kv(b, hkv, t, nb)
+    q = torch.randn((b, hq, 128), generator=g).to(torch.bfloat16).to(DEV)
+    kd = k.to(DEV)
+    kdm = kd.transpose(2, 3).contiguous()
+    score = torch.randint(-9, 9, (b * hq, nb + 3), generator=g).float().to(DEV)   # ties
+    outs = []
+    for select in (True, False):
+        blocks = torch.empty((b * hq, n_scan), dtype=torch.int32, device=DEV)
+        part = torch.empty((b * hq, n_scan * block), dtype=torch.float32, device=DEV)
+        fs = torch.empty_like(part)
+        head = (q.data_ptr(), kdm.data_ptr(), _lib.strides(*kdm.stride()), kd.data_ptr(), _lib.strides(*kd.stride()),
+                b, hq, hkv, t, 128)
+        tail = (n_scan, block, 8, 0.3, part.data_ptr(), fs.data_ptr() if full else None, n_scan * block, 0,
+                _lib.stream_of(q))
+        if select:
+            _lib.check(lib.qkv_block_select_scan_scores(*head, score.data_ptr(), nb + 3, blocks.data_ptr(), *tail))
+        else:
+            BS.block_topk(score[:, :nb], n_scan, out=blocks)
+            _lib.check(lib.qkv_block_scan_scores(*head, blocks.data_ptr(), *tail))
+        outs.append((blocks, part) + ((fs,) if full else ()))
+    for x, y in zip(*outs):
+        assert torch.equal(x, y)
+    assert lib.qkv_block_select_scan_scores(*head, score.data_ptr(), nb + 3, blocks.data_ptr(), nb + 1, *tail[1:]) == -1
