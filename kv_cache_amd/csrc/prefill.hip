@@ -180,9 +180,17 @@ __device__ __forceinline__ v4i unpack_half(uint32_t w0, uint32_t w1) {
 // biased accumulator, below), maximum over the keys a lane holds with
 // v_max3, and at the block end over the 4 row groups with lane swaps.  The
 // LDS copy is double-buffered: block kb+1 is staged while block kb is
-// scored, one workgroup barrier per block.  Only blocks on the causal
-// diagonal or past the last token take the masked epilogue (uniform over
-// the workgroup).
+// scored, one workgroup barrier per block.  The loads run two blocks ahead of
+// their use, in two register sets that the parity of the block selects (one
+// block ahead, a pass of 2048 queries x 65536 tokens, 32/8 heads, took 508 us,
+// now 485-497; a block is scored in less than a load's latency).  All waves load
+// the scales, so that the loads in flight are the same on every path into a
+// wait.  At most two waves per SIMD are asked for at each W: asked for more
+// (8/W), the compiler kept part of the accumulators in AGPRs and copied them
+// for every use at W <= 2 (1405 queries x 18145 tokens, 16/8 heads: the whole
+// pass 98 us, 88.7 without the copies, 87 with the loads two blocks ahead).
+// Only blocks on the causal diagonal or past the last token take the masked
+// epilogue (uniform over the workgroup).
 //
 // Every accumulator starts at the bit pattern of 1.5 * 2^23, so the int32
 // result 0x4B400000 + 16*I read as fp32 is exactly 12582912 + 16*I (|16*I| <
@@ -204,7 +212,7 @@ __device__ __forceinline__ void interleave_step() {
 }
 
 template <int W>
-__global__ __launch_bounds__(64 * W, 8 / W) void prefill_scores_kernel(
+__global__ __launch_bounds__(64 * W, 2) void prefill_scores_kernel(
     const int8_t* __restrict__ q8, const uint8_t* __restrict__ kpacked, const uint16_t* __restrict__ kscales,
     int q_heads, int kv_heads, int nq, int tokens, int64_t capacity, int q_pos0, int nb,
     float* __restrict__ bmax) {
@@ -262,26 +270,28 @@ __global__ __launch_bounds__(64 * W, 8 / W) void prefill_scores_kernel(
   const auto srsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(srow + key0), 0, nblk * kBlock * 2,
                                                        0x00020000);
   const int kvoff = col * (kD / 2) + g * 16;
-  uint4 raw[kTiles];
-  uint32_t sraw = 0;
-  auto gload = [&](int kb) {
+  uint4 raw[2][kTiles];
+  uint32_t sraw[2] = {0, 0};
+  auto gload = [&](int kb, auto pc) {
+    constexpr int P = decltype(pc)::value;
 #pragma unroll
     for (int r = 0; r < kTiles; ++r) {
       const int kt = wave + W * r;
       const auto a = __builtin_amdgcn_raw_buffer_load_b128(krsrc, kvoff + kt * 16 * (kD / 2), kb * kBlock * (kD / 2), 0);
-      raw[r] = uint4{a[0], a[1], a[2], a[3]};
+      raw[P][r] = uint4{a[0], a[1], a[2], a[3]};
     }
-    if (wave == 0) sraw = __builtin_amdgcn_raw_buffer_load_b16(srsrc, 2 * lane, kb * kBlock * 2, 0);
+    sraw[P] = __builtin_amdgcn_raw_buffer_load_b16(srsrc, 2 * lane, kb * kBlock * 2, 0);
   };
-  auto stage = [&](int slot) {
+  auto stage = [&](auto pc) {
+    constexpr int slot = decltype(pc)::value;
 #pragma unroll
     for (int r = 0; r < kTiles; ++r) {
       const int kt = wave + W * r;
-      abuf[slot][kt][0][lane] = unpack_half(raw[r].x, raw[r].y);
-      abuf[slot][kt][1][lane] = unpack_half(raw[r].z, raw[r].w);
+      abuf[slot][kt][0][lane] = unpack_half(raw[slot][r].x, raw[slot][r].y);
+      abuf[slot][kt][1][lane] = unpack_half(raw[slot][r].z, raw[slot][r].w);
     }
     if (wave == 0) {
-      const float s = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(sraw)));
+      const float s = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(sraw[slot])));
       float* e = &sbuf[slot][lane >> 4][(lane >> 2) & 3][lane & 3];
       e[0] = s;
       e[4] = __builtin_fmaf(s, -12582912.0f, 0.0f);
@@ -349,20 +359,24 @@ __global__ __launch_bounds__(64 * W, 8 / W) void prefill_scores_kernel(
       tile[wave][16 * (n0 + g) + col][kb] = __builtin_fmaf(m, 0.0625f, 0.0f);
     }
   };
-  // Stages block kb+1 (its codes were loaded one block earlier) and loads
-  // block kb+2.  Slot (kb+1) % 2 was last read for block kb-1, before the
-  // barrier that ended it.
-  auto stage_next = [&](int kb) {
+  // Block kb (of parity P) stages block kb+1, whose codes were loaded two
+  // blocks earlier, and loads block kb+3 into the same registers.  LDS slot
+  // (kb+1) % 2 was last read for block kb-1, before the barrier that ended it.
+  auto stage_next = [&](int kb, auto pc) {
+    constexpr std::integral_constant<int, 1 - decltype(pc)::value> np{};
     if (kb + 1 < nvis) {
-      stage((kb + 1) & 1);
-      if (kb + 2 < nvis) gload(kb + 2);
+      stage(np);
+      if (kb + 3 < nvis) gload(kb + 3, np);
     }
   };
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
 
   if (nvis > 0) {
-    gload(0);
-    stage(0);
-    if (nvis > 1) gload(1);
+    gload(0, even);
+    if (nvis > 1) gload(1, odd);
+    stage(even);
+    if (nvis > 2) gload(2, even);
     __syncthreads();
   }
   // Unmasked blocks [0, nfull), pipelined by key tile: the MFMAs of tile kt
@@ -377,8 +391,8 @@ __global__ __launch_bounds__(64 * W, 8 / W) void prefill_scores_kernel(
     frag(0, 1, n0, n1, s1, c1);
     mfma_tile(a0, a1, acc0);
   }
-  for (int kb = 0; kb < nfull; ++kb) {
-    const int slot = kb & 1;
+  auto full_block = [&](int kb, auto pc) {
+    constexpr int slot = decltype(pc)::value;
     float4 s2, c2;
     frag(slot, 2, a0, a1, s2, c2);          // prefetch tile 2
     mfma_tile(n0, n1, acc1);                // tile 1
@@ -391,7 +405,7 @@ __global__ __launch_bounds__(64 * W, 8 / W) void prefill_scores_kernel(
     mfma_tile(n0, n1, acc1);                // tile 3
     epi(acc0, s2, c2, false);               // tile 2
     interleave_step();
-    stage_next(kb);
+    stage_next(kb, pc);
     __syncthreads();
     if (kb + 1 < nfull) {
       frag(slot ^ 1, 0, a0, a1, s2, c2);
@@ -406,11 +420,18 @@ __global__ __launch_bounds__(64 * W, 8 / W) void prefill_scores_kernel(
       epi(acc1, s0, c0, false);
       block_end(kb);
     }
+  };
+  int kb = 0;
+  for (; kb + 1 < nfull; kb += 2) {
+    full_block(kb, even);
+    full_block(kb + 1, odd);
   }
+  if (kb < nfull) full_block(kb, even);
   // Blocks [nfull, nvis) hold keys past some query of the tile (the causal
   // diagonal) or past the last token: masked, one tile at a time.
-  for (int kb = nfull; kb < nvis; ++kb) {
-    const int slot = kb & 1, base = (blk0 + kb) * kBlock;
+  auto masked_block = [&](int kb, auto pc) {
+    constexpr int slot = decltype(pc)::value;
+    const int base = (blk0 + kb) * kBlock;
     v4i a0, a1;
     float4 s0, c0;
 #pragma unroll
@@ -420,10 +441,16 @@ __global__ __launch_bounds__(64 * W, 8 / W) void prefill_scores_kernel(
       epi_masked(acc0, s0, c0, kt, base);
     }
     block_end(kb);
-    stage_next(kb);
+    stage_next(kb, pc);
     __syncthreads();
+  };
+  for (kb = nfull; kb < nvis; ++kb) {
+    if (kb & 1)
+      masked_block(kb, odd);
+    else
+      masked_block(kb, even);
   }
-  for (int kb = nvis; kb < nblk; ++kb) {
+  for (kb = nvis; kb < nblk; ++kb) {
     if (lane < 16) {
 #pragma unroll
       for (int n = 0; n < kNT; ++n) tile[wave][16 * n + col][kb] = ninf;
