@@ -346,7 +346,7 @@ def run_decode(args, name: str, layers: int | None = None, with_cpu: bool = True
         for _ in range(layers):
             K.block_topk(step.bmax, cfg.topk, out=step.sel, workspace=step.topk_ws)
 
-    def run_decode_topk():   # the step's token selection: scoring that also builds the top-k's chunk windows
+    def run_decode_topk():   # the step's token selection: scoring that also counts the top-k's row histograms
         for layer in range(layers):
             c = caches[layer]
             K.decode_topk(qs[layer], c.chan_idx, c.slab, c.slab_scales, T, cfg.topk, scores=step.bmax,

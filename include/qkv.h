@@ -203,16 +203,22 @@ int qkv_topk(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k
              int32_t* out, void* stream);
 
 /* Bytes of workspace qkv_topk_ws needs: 0 when qkv_topk's one workgroup per
- * row is used (n <= 4096 or k > 1024); for rows of at most 64 chunks of 4096
- * keys with ceil(n/4096) * k <= 32768, per chunk a 66-word histogram window
- * and a list of k (value, index) pairs with its count; otherwise two
- * candidate buffers of rows * (k * ceil(n/4096)) (value, index) pairs and
+ * row is used (n <= 4096, or n > 196608 with k > 1024); for n <= 196608 a
+ * 4096-bin histogram, a bitset and the slices' lists per row; otherwise (and
+ * never less than) what the chunk lists below take: for rows of at most 64
+ * chunks of 4096 keys with ceil(n/4096) * k <= 32768, per chunk a 66-word
+ * histogram window and a list of k (value, index) pairs with its count, else
+ * two candidate buffers of rows * (k * ceil(n/4096)) (value, index) pairs and
  * rows * ceil(n/4096) uint32 chunk bounds; -1 for bad sizes. */
 int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k);
 
 /* qkv_topk with a caller-owned workspace (16-byte aligned, contents
- * irrelevant; calls sharing a workspace must not overlap in time): rows
- * longer than 4096 keys with k <= 1024 are split into 4096-key chunks.  Rows
+ * irrelevant; calls sharing a workspace must not overlap in time).  Rows of
+ * 4097 to 196608 keys, any k: three launches clear a histogram per row, count
+ * the keys' top 12 bits into it, and select from slices of the row.  With
+ * k <= 1024, longer rows, and calls with a workspace smaller than
+ * qkv_topk_workspace_bytes but enough for the chunk lists, are split into
+ * 4096-key chunks; with k > 1024 such calls take qkv_topk.  Rows
  * of at most 64 chunks with chunks * k <= 32768: every chunk histograms its
  * keys (1/8-octave bins) around its own k-th key, the row's floor is the bin
  * where the merged count from the top reaches k, each chunk keeps its keys
@@ -237,10 +243,10 @@ int qkv_topk_ws(const float* values, int64_t rows, int64_t n, int64_t ld, int64_
  * block 1 into scores f32 [batch * kv_heads, tokens], then qkv_topk_ws over
  * those rows into out int32 [rows, k] (the same result as the two calls).
  * workspace: qkv_topk_workspace_bytes(rows, tokens, k) bytes, 16-byte
- * aligned, contents irrelevant.  Where qkv_topk_ws takes its
- * histogram-and-filter path, the scoring launch (one workgroup per
- * 4096-token chunk) also builds each chunk's histogram window, so the top-k
- * starts at the row's floor.  Replaces the reference's partial scores plus
+ * aligned, contents irrelevant.  Where qkv_topk_ws selects from a row
+ * histogram or from chunk lists with histogram windows, the scoring launch
+ * (one workgroup per 4096-token chunk) counts the keys as it scores, so the
+ * top-k needs no pass of its own for that.  Replaces the reference's partial scores plus
  * torch.topk at EV:5038-5046 for block 1 (no counterpart as one call). */
 int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
                          const int32_t* chan_idx, int64_t selected, const uint8_t* slab,

@@ -581,7 +581,7 @@ __global__ __launch_bounds__(kRT) void final_from_selected_kernel(
 // ---------------------------------------------------------------------------
 // Rows of at most kWideMax values: one 1024-thread workgroup per row holds
 // the row in registers (WideSelect) and does the whole selection in one
-// launch.  Longer rows take the staged top-k and the kernels above.
+// launch.  Longer rows take the long-row top-k and the kernels above.
 // ---------------------------------------------------------------------------
 constexpr int kWideNT = 1024;
 constexpr int kWideMax = kWideNT * 40;
@@ -1836,7 +1836,9 @@ int with_wide_vpl(int64_t n, F&& f) {
 // The same in finer steps, for kernels that always work on the whole row: a
 // wave owns 64 * VPL consecutive positions, so a row a little longer than a
 // coarse step would leave half the workgroup's waves without keys and give
-// the others twice as many.
+// the others twice as many: 128 rows of 16410 scores at 32 values a thread
+// 21.4 us, at 20 18.6; exact candidate attention over 256 rows of 4000 at 16
+// 42.5 us a layer, at 4 38.9.
 template <typename F>
 int with_wide_vpl_fine(int64_t n, F&& f) {
   if (n <= 4 * kWideNT) return f(std::integral_constant<int, 4>{});
@@ -1909,7 +1911,7 @@ int64_t block_body_cap(const ReuseCounts& c, int64_t block) {
 
 constexpr int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
-// Scores, selection, staged top-k workspace, then (rows the wide kernel
+// Scores, selection, long-row top-k workspace, then (rows the wide kernel
 // selects in one workgroup) the compacted union lists and their counts.
 int64_t reuse_compact_bytes(int64_t rows, int64_t history) {
   if (history > kWideMax) return 0;

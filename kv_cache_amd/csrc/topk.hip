@@ -1,5 +1,7 @@
 // Row-wise top-k with the lowest-index tie-break: one workgroup per row, or,
-// for long rows, a staged reduction over 4096-key chunks (topk_stage_kernel).
+// for long rows, a row histogram and slices of the row (topk_slices_kernel);
+// rows past kBigMax, and calls whose workspace holds no histogram, take lists
+// of 4096-key chunks (topk_fused_kernel, topk_stage_kernel).
 //
 // The reference calls torch.topk over partial scores or block maxima
 // (evaluate_qwen3_top2_head_limit3_ppl.py:4448, 5046), whose tie order is

@@ -200,8 +200,8 @@ def decode_topk(query: torch.Tensor, chan_idx: torch.Tensor, slab: torch.Tensor,
     """``decode_scores`` with block 1 then ``block_topk`` in one call
     (qkv_int4_decode_topk): the top-k token indices int32 [B, Hkv, k],
     ascending, lowest index first among equal scores; the token scores go to
-    ``scores`` f32 [B, Hkv, tokens].  Long rows build the top-k's chunk
-    histograms while they score.  ``state`` (from ``topk_state``) is kept zero
+    ``scores`` f32 [B, Hkv, tokens].  Long rows count the top-k's row
+    histogram while they score.  ``state`` (from ``topk_state``) is kept zero
     from call to call and saves the launch that clears it."""
     lib = _lib.load()
     code = _check_query(query)
@@ -251,7 +251,7 @@ def topk_workspace(rows: int, n: int, k: int, device) -> torch.Tensor | None:
 def block_topk(values: torch.Tensor, k: int, *, out: torch.Tensor | None = None,
                workspace: torch.Tensor | None = None) -> torch.Tensor:
     """Top-k indices along the last axis, lowest index wins ties, ascending order (int32).
-    Rows longer than 4096 values use a staged selection with a workspace
+    Rows longer than 4096 values are selected by many workgroups each, with a workspace
     (allocated here unless one from ``topk_workspace`` is passed)."""
     lib = _lib.load()
     _require(values.is_cuda and values.dtype == torch.float32, "values must be CUDA float32")
@@ -522,7 +522,7 @@ class SparseDecodeStep:
                           bmax=self.bmax)
             return sparse_attention_select(query, key, value, self.bmax, self.topk, self.block, self.scored,
                                            scaling, workspace=self.workspace, sel_out=self.sel, out=self.out, **prot)
-        if self.block == 1:   # token selection: the scoring launch feeds the top-k its chunk histograms
+        if self.block == 1:   # token selection: the scoring launch feeds the top-k its row histograms
             decode_topk(query, cache.chan_idx, cache.slab, cache.slab_scales, self.scored, self.topk,
                         scores=self.bmax, out=self.sel, workspace=self.topk_ws, state=self.topk_state)
         else:
