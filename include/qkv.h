@@ -202,22 +202,27 @@ int qkv_int4_decode_scores(const void* query, int64_t batch, int64_t q_heads, in
 int qkv_topk(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k,
              int32_t* out, void* stream);
 
-/* Bytes of workspace qkv_topk_ws needs: 0 when qkv_topk's one workgroup per
- * row is used (n <= 4096, or n > 196608 with k > 1024); for n <= 196608 a
- * 4096-bin histogram, a bitset and the slices' lists per row; otherwise (and
- * never less than) what the chunk lists below take: for rows of at most 64
- * chunks of 4096 keys with ceil(n/4096) * k <= 32768, per chunk a 66-word
- * histogram window and a list of k (value, index) pairs with its count, else
- * two candidate buffers of rows * (k * ceil(n/4096)) (value, index) pairs and
- * rows * ceil(n/4096) uint32 chunk bounds; -1 for bad sizes. */
+/* Bytes of workspace for qkv_topk_ws on rows of n keys: enough for n and for
+ * every shorter row with the same or a smaller k, so a workspace sized once
+ * for the longest row serves them all (the size functions below that are
+ * built on it hold to the same for a shorter history).  0 for n <= 4096; for
+ * n <= 196608 a 4096-bin histogram, a bitset and the slices' lists per row,
+ * whatever k; past that no less than this for 196608 and what the chunk lists
+ * below take: for rows of at most 64 chunks of 4096 keys with ceil(n/4096) * k
+ * <= 32768, per chunk a 66-word histogram window and a list of k (value,
+ * index) pairs with its count, else two candidate buffers of rows * (k *
+ * ceil(n/4096)) (value, index) pairs and rows * ceil(n/4096) uint32 chunk
+ * bounds; -1 for bad sizes.  A call with k <= 1024 is refused only where its
+ * workspace holds neither the row histogram nor the chunk lists of its n and
+ * k. */
 int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k);
 
 /* qkv_topk with a caller-owned workspace (16-byte aligned, contents
  * irrelevant; calls sharing a workspace must not overlap in time).  Rows of
  * 4097 to 196608 keys, any k: three launches clear a histogram per row, count
  * the keys' top 12 bits into it, and select from slices of the row.  With
- * k <= 1024, longer rows, and calls with a workspace smaller than
- * qkv_topk_workspace_bytes but enough for the chunk lists, are split into
+ * k <= 1024, longer rows, and calls with a workspace smaller than the row
+ * histogram's but enough for the chunk lists, are split into
  * 4096-key chunks; with k > 1024 such calls take qkv_topk.  Rows
  * of at most 64 chunks with chunks * k <= 32768: every chunk histograms its
  * keys (1/8-octave bins) around its own k-th key, the row's floor is the bin

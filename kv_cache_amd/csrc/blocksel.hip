@@ -747,9 +747,10 @@ bool rerank_fits(int64_t history, int64_t n_scan, int64_t block, int64_t n_cand,
 
 // Workspace of the general rerank: dense scores [rows, dense_ld], candidate
 // tokens and their full scores [rows, n1], kept indices [rows, n2], then the
-// top-k workspace shared by both selections; 256-byte aligned parts.
+// top-k workspace shared by both selections; 256-byte aligned parts.  least:
+// what a call must bring; total: what the size function returns.
 struct WideRerank {
-  int64_t dense_ld, n1, n2, off_cand, off_cf, off_kept, off_topk, topk_bytes, total;
+  int64_t dense_ld, n1, n2, off_cand, off_cf, off_kept, off_topk, least, total;
 };
 
 WideRerank wide_rerank_layout(int64_t rows, int64_t history, int64_t n_cand, int64_t n_keep) {
@@ -766,8 +767,9 @@ WideRerank wide_rerank_layout(int64_t rows, int64_t history, int64_t n_cand, int
   w.off_kept = off;
   off += al(rows * w.n2 * 4);
   w.off_topk = off;
-  w.topk_bytes = std::max(qkv_topk_workspace_bytes(rows, history, w.n1), qkv_topk_workspace_bytes(rows, w.n1, w.n2));
-  w.total = off + al(std::max<int64_t>(w.topk_bytes, 0));
+  auto end = [&](int64_t first, int64_t second) { return off + al(std::max<int64_t>({first, second, 0})); };
+  w.least = end(topk_least_bytes(rows, history, w.n1), topk_least_bytes(rows, w.n1, w.n2));
+  w.total = end(qkv_topk_workspace_bytes(rows, history, w.n1), qkv_topk_workspace_bytes(rows, w.n1, w.n2));
   return w;
 }
 
@@ -1044,21 +1046,22 @@ QKV_EXPORT int qkv_block_rerank(const void* query, const void* key, const int64_
   const int rows = static_cast<int>(batch * q_heads);
   if (!rerank_fits(history, n_scan, block, n_cand, unscanned != 0)) {
     const WideRerank w = wide_rerank_layout(rows, history, n_cand, n_keep);
-    if (!workspace || !aligned(workspace, 256) || workspace_bytes < w.total)
+    if (!workspace || !aligned(workspace, 256) || workspace_bytes < w.least)
       return fail(QKV_ERR_INVALID, "%s: this rerank needs a 256-byte aligned workspace of %lld bytes, got %lld",
-                  what, (long long)w.total, (long long)workspace_bytes);
+                  what, (long long)w.least, (long long)workspace_bytes);
     char* ws = static_cast<char*>(workspace);
     float* dense = reinterpret_cast<float*>(ws);
     int32_t* cand = reinterpret_cast<int32_t*>(ws + w.off_cand);
     float* cf = reinterpret_cast<float*>(ws + w.off_cf);
     int32_t* kept = reinterpret_cast<int32_t*>(ws + w.off_kept);
     void* tws = ws + w.off_topk;
+    const int64_t tws_bytes = workspace_bytes - w.off_topk;
     const float fill = unscanned ? -3.40282347e38f : -__builtin_huge_valf();   // finfo(float32).min / -inf
     dense_partial_kernel<<<dim3(static_cast<unsigned>(cdiv(history, kBT)), rows), kBT, 0, st>>>(
         partial, partial_ld, blocks, static_cast<int>(n_scan), static_cast<int>(block), static_cast<int>(history),
         fill, dense, w.dense_ld);
     if ((rc = check_launch(what))) return rc;
-    if ((rc = qkv_topk_ws(dense, rows, history, w.dense_ld, w.n1, cand, tws, w.topk_bytes, stream))) return rc;
+    if ((rc = qkv_topk_ws(dense, rows, history, w.dense_ld, w.n1, cand, tws, tws_bytes, stream))) return rc;
     rc = with_half(f16, [&](auto ff) {
       cand_full_kernel<decltype(ff)::value><<<dim3(static_cast<unsigned>(cdiv(w.n1, kBT)), rows), kBT, 0, st>>>(
           static_cast<const uint16_t*>(query), static_cast<const uint16_t*>(key), static_cast<int>(q_heads),
@@ -1067,7 +1070,7 @@ QKV_EXPORT int qkv_block_rerank(const void* query, const void* key, const int64_
       return check_launch(what);
     });
     if (rc) return rc;
-    if ((rc = qkv_topk_ws(cf, rows, w.n1, w.n1, w.n2, kept, tws, w.topk_bytes, stream))) return rc;
+    if ((rc = qkv_topk_ws(cf, rows, w.n1, w.n1, w.n2, kept, tws, tws_bytes, stream))) return rc;
     rerank_finish_kernel<<<static_cast<unsigned>(rows), kRerankNT, 0, st>>>(
         cand, cf, static_cast<int>(w.n1), kept, static_cast<int>(w.n2), static_cast<int>(n_keep),
         static_cast<int>(history), static_cast<int>(key_count), static_cast<int>(sink_end),

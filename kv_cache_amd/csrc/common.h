@@ -21,6 +21,10 @@ int check_launch(const char* what);
 inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// The least workspace qkv_topk_ws runs with (topk.hip); what
+// qkv_topk_workspace_bytes returns is larger.
+int64_t topk_least_bytes(int64_t rows, int64_t n, int64_t k);
+
 // Resolves the dtype of a 16-bit operand (query, K, V): sets *f16 (false for
 // bf16, true for fp16) and returns QKV_OK, or fails for fp32 and unknown codes.
 inline int half_dtype(int dtype, const char* what, bool* f16) {

@@ -777,7 +777,6 @@ int topk_filtered(const float* values, int64_t rows, int64_t n, int64_t ld, int6
                   void* workspace, hipStream_t st, bool given);
 bool topk_takes_windows(int64_t n, int64_t k);
 bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes);
-int64_t topk_least_bytes(int64_t rows, int64_t n, int64_t k);
 int64_t topk_hist_stride();
 int topk_big_clear(int64_t rows, int64_t n, void* workspace, hipStream_t st, int** hist, int64_t* stride);
 int topk_big_finish(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,

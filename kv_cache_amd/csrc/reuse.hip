@@ -1911,24 +1911,39 @@ int64_t block_body_cap(const ReuseCounts& c, int64_t block) {
 
 constexpr int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
-// Scores, selection, long-row top-k workspace, then (rows the wide kernel
-// selects in one workgroup) the compacted union lists and their counts.
+// Scores, selection, then the long-row top-k's workspace or (rows the wide
+// kernel selects in one workgroup) the compacted union lists and their counts.
 int64_t reuse_compact_bytes(int64_t rows, int64_t history) {
   if (history > kWideMax) return 0;
   const int64_t slots = cdiv(history, kScoreTile) * kScoreTile;
   return 2 * align256(rows * slots * 4) + align256(rows * cdiv(history, kScoreTile) * 2 * 4);
 }
 
+// `reuse_need`: what a call at this history uses at least.  `reuse_ws_bytes`:
+// enough for it and for every shorter history with no larger keep (a step
+// sizes its workspace once, for its capacity).  Likewise below: *_need is
+// checked against, *_bytes is what the size functions return.
+int64_t reuse_need(int64_t rows, int64_t history, int64_t keep) {
+  const int64_t base = align256(rows * history * 4) + align256(rows * keep * 4);
+  if (history <= kWideMax) return base + reuse_compact_bytes(rows, history);
+  const int64_t tk = topk_least_bytes(rows, history, keep);
+  return tk < 0 ? -1 : base + align256(tk);
+}
 int64_t reuse_ws_bytes(int64_t rows, int64_t history, int64_t keep) {
+  const int64_t wide = std::min<int64_t>(history, kWideMax);
+  const int64_t one = align256(rows * wide * 4) + align256(rows * keep * 4) + reuse_compact_bytes(rows, wide);
+  if (history <= kWideMax) return one;
   const int64_t tk = qkv_topk_workspace_bytes(rows, history, keep);
-  if (tk < 0) return -1;
-  return align256(rows * history * 4) + align256(rows * keep * 4) + align256(tk) + reuse_compact_bytes(rows, history);
+  return tk < 0 ? -1 : std::max(one, align256(rows * history * 4) + align256(rows * keep * 4) + align256(tk));
 }
 
+int64_t mask_need(int64_t rows, int64_t n, int64_t k) {
+  const int64_t tk = topk_least_bytes(rows, n, k);
+  return tk < 0 ? -1 : align256(rows * k * 4) + align256(tk);
+}
 int64_t mask_ws_bytes(int64_t rows, int64_t n, int64_t k) {
   const int64_t tk = qkv_topk_workspace_bytes(rows, n, k);
-  if (tk < 0) return -1;
-  return align256(rows * k * 4) + align256(tk);
+  return tk < 0 ? -1 : align256(rows * k * 4) + align256(tk);
 }
 
 // hist (optional, [B * Hq, kCandBins] int, zero): every row's first-digit
@@ -2043,9 +2058,12 @@ int64_t cand_state_bytes(int64_t rows) { return align256(rows * kCandBins * 4) +
 
 // The rest of the workspace: the boundary-bin lists (a score and a position
 // per history token and row) or, on the other paths, qkv_threshold_mask's.
-int64_t cand_scratch_bytes(int64_t rows, int64_t n, int64_t k) {
-  const int64_t m = mask_ws_bytes(rows, n, k);
-  return m < 0 ? -1 : std::max(m, 2 * align256(rows * n * 4));
+int64_t cand_scratch(int64_t rows, int64_t n, int64_t mask_bytes) {
+  return mask_bytes < 0 ? -1 : std::max(mask_bytes, 2 * align256(rows * n * 4));
+}
+int64_t cand_need(int64_t rows, int64_t n, int64_t k) {
+  const int64_t scratch = cand_scratch(rows, n, mask_need(rows, n, k));
+  return scratch < 0 ? -1 : cand_state_bytes(rows) + scratch;
 }
 
 struct CandSplit {
@@ -2222,7 +2240,7 @@ int reuse_select_impl(const char* what, bool bits, const void* query, const void
                 (long long)n_out, (long long)c.n_out);
   }
   const int64_t rows = batch * q_heads;
-  const int64_t need = reuse_ws_bytes(rows, history, c.keep);
+  const int64_t need = reuse_need(rows, history, c.keep);
   if (need < 0 || workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
@@ -2232,9 +2250,6 @@ int reuse_select_impl(const char* what, bool bits, const void* query, const void
   int64_t off = align256(rows * history * 4);
   int32_t* sel = reinterpret_cast<int32_t*>(ws + off);
   off += align256(rows * c.keep * 4);
-  void* tk_ws = ws + off;
-  const int64_t tk_bytes = align256(qkv_topk_workspace_bytes(rows, history, c.keep));
-  off += tk_bytes;
   const bool wide = history <= kWideMax;
   const int64_t n_tiles = cdiv(history, kScoreTile), c_ld = n_tiles * kScoreTile;
   float* cscore = wide ? reinterpret_cast<float*>(ws + off) : nullptr;
@@ -2282,7 +2297,7 @@ int reuse_select_impl(const char* what, bool bits, const void* query, const void
                   : launch(std::false_type{}, BF{}, std::false_type{});
     });
   }
-  rc = qkv_topk_ws(scores, rows, history, history, c.keep, sel, tk_ws, tk_bytes, stream);
+  rc = qkv_topk_ws(scores, rows, history, history, c.keep, sel, ws + off, workspace_bytes - off, stream);
   if (rc) return rc;
   auto fin = [&](auto bb) {
     reuse_finalize_kernel<decltype(bb)::value><<<static_cast<unsigned>(rows), kRT, 0, st>>>(
@@ -2385,7 +2400,7 @@ QKV_EXPORT int qkv_qabs_candidate_select(const float* scores, int64_t rows, int6
       return check_launch(what);
     });
   }
-  const int64_t need = mask_ws_bytes(rows, history, c.keep);
+  const int64_t need = mask_need(rows, history, c.keep);
   if (!workspace || need < 0 || workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
@@ -2403,10 +2418,9 @@ QKV_EXPORT int qkv_qabs_candidate_select(const float* scores, int64_t rows, int6
 }
 
 QKV_EXPORT int64_t qkv_qabs_candidates_workspace_bytes(int64_t rows, int64_t history, double candidate_fraction) {
-  const int64_t old = qkv_qabs_candidate_select_workspace_bytes(rows, history, candidate_fraction);
-  if (old < 0) return -1;
-  const int64_t split = history <= kWideMax ? qabs_split_bytes(rows, history) : 0;
-  return cand_state_bytes(rows) + std::max(old, split);
+  const int64_t select = qkv_qabs_candidate_select_workspace_bytes(rows, history, candidate_fraction);
+  if (select < 0) return -1;
+  return cand_state_bytes(rows) + std::max(select, qabs_split_bytes(rows, std::min<int64_t>(history, kWideMax)));
 }
 
 QKV_EXPORT int qkv_qabs_candidates(const void* query, const void* key_dim_major, const int64_t* kdm_strides, int dtype,
@@ -2433,8 +2447,9 @@ QKV_EXPORT int qkv_qabs_candidates(const void* query, const void* key_dim_major,
   if (n_out != c.n_out)
     return fail(QKV_ERR_INVALID, "%s: index rows hold %lld entries, the selection needs %lld", what,
                 (long long)n_out, (long long)c.n_out);
-  const int64_t need = qkv_qabs_candidates_workspace_bytes(rows, history, candidate_fraction);
-  if (need < 0 || workspace_bytes < need)
+  const int64_t scratch = history <= kWideMax ? qabs_split_bytes(rows, history) : mask_need(rows, history, c.keep);
+  const int64_t need = cand_state_bytes(rows) + scratch;
+  if (scratch < 0 || workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
   if (!aligned(workspace, 16)) return fail(QKV_ERR_INVALID, "%s: the workspace must be 16-byte aligned", what);
@@ -2601,7 +2616,7 @@ QKV_EXPORT int qkv_threshold_mask(const float* values, int64_t rows, int64_t n, 
   if (!values || !mask || !workspace) return fail(QKV_ERR_INVALID, "%s: null pointer", what);
   if (rows <= 0 || rows > 65535 || n <= 0 || n >= (int64_t(1) << 31) || k < 1 || k > n || ld < n || mask_ld < n)
     return fail(QKV_ERR_INVALID, "%s: need 0 < rows <= 65535, 1 <= k <= n, ld and mask_ld >= n", what);
-  const int64_t need = mask_ws_bytes(rows, n, k);
+  const int64_t need = mask_need(rows, n, k);
   if (need < 0 || workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
@@ -2628,7 +2643,7 @@ QKV_EXPORT int qkv_reuse_lag_candidates(const void* query, const void* key_dim_m
     return fail(QKV_ERR_INVALID, "%s: unknown refresh %d", what, refresh);
   if (refresh >= QKV_REFRESH_PER_ROW && !flags) return fail(QKV_ERR_INVALID, "%s: null flags", what);
   const int64_t rows = batch * q_heads;
-  const int64_t need = mask_ws_bytes(rows, history, k);
+  const int64_t need = mask_need(rows, history, k);
   if (need < 0 || workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
@@ -2661,7 +2676,7 @@ QKV_EXPORT int qkv_reuse_lag_candidates_bits(const void* query, const void* key_
     return fail(QKV_ERR_INVALID, "%s: unknown refresh %d", what, refresh);
   if (refresh >= QKV_REFRESH_PER_ROW && !flags) return fail(QKV_ERR_INVALID, "%s: null flags", what);
   const int64_t rows = batch * q_heads;
-  const int64_t need = qkv_reuse_candidates_workspace_bytes(rows, history, k);
+  const int64_t need = cand_need(rows, history, k);
   if (need < 0 || workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
@@ -2700,7 +2715,7 @@ QKV_EXPORT int qkv_reuse_candidates(const void* query, const void* key_dim_major
                 what);
   if (kdm_strides[3] != 1) return fail(QKV_ERR_UNSUPPORTED, "%s: the token axis of K must be contiguous", what);
   const int64_t rows = batch * q_heads;
-  const int64_t need = qkv_reuse_candidates_workspace_bytes(rows, history, k);
+  const int64_t need = cand_need(rows, history, k);
   if (need < 0 || workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
@@ -2722,7 +2737,7 @@ QKV_EXPORT int qkv_reuse_candidates(const void* query, const void* key_dim_major
 
 QKV_EXPORT int64_t qkv_reuse_candidates_workspace_bytes(int64_t rows, int64_t history, int64_t k) {
   if (rows <= 0 || history <= 0 || history >= (int64_t(1) << 31) || k < 1 || k > history) return -1;
-  const int64_t scratch = cand_scratch_bytes(rows, history, k);
+  const int64_t scratch = cand_scratch(rows, history, mask_ws_bytes(rows, history, k));
   return scratch < 0 ? -1 : cand_state_bytes(rows) + scratch;
 }
 
@@ -2750,7 +2765,7 @@ QKV_EXPORT int qkv_candidate_mask(const float* values, int64_t rows, int64_t n, 
   if (selection == QKV_CAND_TOPK) {
     if (k < 1 || k > n) return fail(QKV_ERR_INVALID, "%s: need 1 <= k <= n", what);
     if (!workspace) return fail(QKV_ERR_INVALID, "%s: null pointer", what);
-    const int64_t need = mask_ws_bytes(rows, n, k);
+    const int64_t need = mask_need(rows, n, k);
     if (need < 0 || workspace_bytes < need)
       return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                   (long long)workspace_bytes);
@@ -2773,8 +2788,9 @@ QKV_EXPORT int qkv_candidate_mask(const float* values, int64_t rows, int64_t n, 
   if (!sample_cols || !workspace) return fail(QKV_ERR_INVALID, "%s: null pointer", what);
   if (n_sample < 1 || n_sample > n || k < 1 || k > n_sample)
     return fail(QKV_ERR_INVALID, "%s: need 1 <= k <= n_sample <= n", what);
-  const int64_t need = qkv_candidate_mask_workspace_bytes(rows, n, selection, k, n_sample);
-  if (need < 0 || workspace_bytes < need)
+  const int64_t kth = n_sample <= kWideMax ? 0 : mask_need(rows, n_sample, k);
+  const int64_t need = align256(rows * n_sample * 4) + kth;
+  if (kth < 0 || workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
   if (n_sample <= kRT) {   // gather, k-th of the sample and compare in one launch

@@ -1743,8 +1743,12 @@ static int64_t staged_bytes(int64_t rows, int64_t n, int64_t k) {
 
 int64_t topk_hist_stride() { return kBigStride; }
 
+// The least workspace a call of these sizes runs with: the row histogram's or
+// the chunk lists', whichever is smaller (-1: bad sizes).
 int64_t topk_least_bytes(int64_t rows, int64_t n, int64_t k) {
-  return rows <= 0 || n <= 0 || k < 1 || k > n ? -1 : staged_bytes(rows, n, k);
+  if (rows <= 0 || n <= 0 || k < 1 || k > n) return -1;
+  const int64_t lists = staged_bytes(rows, n, k);
+  return big(n) && rows <= 65535 ? std::min(lists, big_ws(nullptr, rows, n).bytes) : lists;
 }
 
 // Whether a call takes the row-histogram path: its sizes, and a workspace that holds it.
@@ -1759,9 +1763,19 @@ QKV_EXPORT int64_t qkv_topk_state_bytes(int64_t rows, int64_t n, int64_t k) {
   return big(n) && rows <= 65535 ? big_state_bytes(rows) : 0;
 }
 
+// Enough for (n, k) and for every shorter row with no larger k, so that a
+// workspace sized once for the longest row is never too small: the row
+// histogram's bytes grow with n up to kBigMax, whatever k; past it the chunk
+// lists' grow with n and k except where n passes kFilterMaxChunks chunks
+// (smaller lists, without windows) and where k passes kStageMaxK (no lists).
 QKV_EXPORT int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
   if (rows <= 0 || n <= 0 || k < 1 || k > n) return -1;
-  return std::max(staged_bytes(rows, n, k), big(n) && rows <= 65535 ? big_ws(nullptr, rows, n).bytes : int64_t{0});
+  if (rows > 65535 || n <= kStageChunk) return staged_bytes(rows, n, k);
+  const int64_t hist = big_ws(nullptr, rows, std::min(n, kBigMax)).bytes;
+  if (n <= kBigMax) return hist;
+  const int64_t kl = std::min<int64_t>(k, kStageMaxK);
+  const int64_t windows_end = std::min<int64_t>(n, kFilterMaxChunks * kStageChunk);
+  return std::max({hist, staged_bytes(rows, n, kl), staged_bytes(rows, windows_end, kl)});
 }
 
 QKV_EXPORT int qkv_topk_ws(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
@@ -1773,7 +1787,7 @@ QKV_EXPORT int qkv_topk_ws(const float* values, int64_t rows, int64_t n, int64_t
     return fail(QKV_ERR_INVALID, "qkv_topk_ws: bad sizes rows=%lld n=%lld ld=%lld", (long long)rows,
                 (long long)n, (long long)ld);
   const int64_t need = staged_bytes(rows, n, k);
-  if (workspace_bytes < need)
+  if (!row_hist && workspace_bytes < need)
     return fail(QKV_ERR_INVALID, "qkv_topk_ws: workspace needs %lld bytes, got %lld", (long long)need,
                 (long long)workspace_bytes);
   if (!aligned(workspace, 16)) return fail(QKV_ERR_INVALID, "qkv_topk_ws: workspace must be 16-byte aligned");

@@ -251,3 +251,45 @@ def test_qabs_candidates_equal_two_calls(b, hist, pattern, frac, sink, recent, k
     if pattern == "equal":
         keep = want[0].size(1) - (sink + recent + keep_self)
         assert torch.equal(got[0][:, :keep].cpu(), torch.arange(keep).expand(rows, keep))
+
+
+def test_step_at_histories_far_below_its_capacity():
+    # the workspace is sized once, at the capacity: every shorter history, on each of the selection's
+    # paths (one workgroup a row, row histogram, past it), runs on it and selects as a step of its own size
+    cap, frac = 262145, 0.03
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    k = torch.randn((1, 2, cap, 128), generator=gen, device=DEV).to(torch.bfloat16)
+    v = torch.randn((1, 2, cap, 128), generator=gen, device=DEV).to(torch.bfloat16)
+    step = RU.QabsCandidateAttentionStep("qabs8cand3attn", 1, 8, 2, 128, cap, protect_sink=4, protect_recent=16)
+    held = step.sel_ws.data_ptr()
+    for hist in (4000, 30000, 65536, 196608, 200001, cap - 1):
+        q = torch.randn((1, 8, 128), generator=gen, device=DEV).to(torch.bfloat16)
+        out = step(q, k[:, :, : hist + 1], v[:, :, : hist + 1], 128 ** -0.5).clone()
+        assert step.sel_ws.data_ptr() == held
+        own = RU.QabsCandidateAttentionStep("qabs8cand3attn", 1, 8, 2, 128, hist + 1, protect_sink=4,
+                                            protect_recent=16)
+        assert torch.equal(out, own(q, k[:, :, : hist + 1], v[:, :, : hist + 1], 128 ** -0.5))
+        keep = RU.budget_count(hist, frac)
+        want = topk_lowest_index(f32(step.partial[:, :hist]), keep)
+        assert np.array_equal(np.sort(step.final_indices()[0][0, :, :keep].cpu().numpy()), want)
+
+
+@pytest.mark.parametrize("hist,frac", [(65536, 0.03), (100001, 0.02), (50000, 0.01)])
+def test_candidate_select_with_the_least_workspace(hist, frac):
+    # with k > 1024 the selection needs only the k indices a row; with fewer the chunk lists' bytes also do
+    from kv_cache_amd import _lib
+
+    lib = _lib.load()
+    scores = torch.randn((4, hist), generator=torch.Generator().manual_seed(hist)).to(DEV)
+    want = RU.qabs_candidate_select(scores, hist + 1, frac, 4, 16, True)
+    keep, chunks = RU.budget_count(hist, frac), -(-hist // 4096)
+    lists = 0 if keep > 1024 else 4 * chunks * (66 + 2 * keep + 1) * 4
+    need = -(-(4 * keep * 4) // 256) * 256 + -(-lists // 256) * 256
+    assert need < lib.qkv_qabs_candidate_select_workspace_bytes(4, hist, frac)
+    ws = torch.empty(need // 4, device=DEV)
+    got = tuple(torch.zeros_like(w) for w in want)
+    _lib.check(lib.qkv_qabs_candidate_select(
+        scores.data_ptr(), 4, hist + 1, hist, frac, 4, 16, 1, 0, ws.data_ptr(), need, got[0].data_ptr(),
+        got[1].data_ptr(), got[2].data_ptr(), got[0].size(1), got[3].data_ptr(), hist, _lib.stream_of(scores)))
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
