@@ -82,15 +82,6 @@ __device__ __forceinline__ uint32_t f32_to_f16bits_sat(float x) {
   return bits == 0x7C00u ? 0x7BFFu : bits;
 }
 
-// Symmetric int4 code of x for an fp16-representable scale s (s > 0):
-// clamp(rint_even(x / s), -8, 7).  The division is the IEEE-correct one
-// (hipcc's default for fp32 '/').
-__device__ __forceinline__ int int4_code(float x, float s) {
-  float r = __builtin_rintf(x / s);
-  r = fminf(fmaxf(r, -8.0f), 7.0f);
-  return static_cast<int>(r);
-}
-
 // Order-preserving map of an fp32 key onto uint32 (larger float -> larger
 // integer), with -0 folded onto +0.  NaN inputs are outside the contract.
 __device__ __forceinline__ uint32_t f32_sortable(float f) {

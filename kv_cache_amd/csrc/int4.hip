@@ -68,7 +68,9 @@ __device__ __forceinline__ float code_rcp(float s) { return s != 0.0f ? __builti
 // 0x4B400000 + code in the bits; the codes are gathered by shift-and-add
 // (the constants' sum is known) as (code + 8) nibbles, then xor 8.  4.3
 // instructions a value; the IEEE division with rint, conversion and masking
-// took about 20 and bound the pack kernel.
+// took about 20 and bound the pack kernel.  The scale 0 (rs = 0) gives code 0
+// for every value, and a NaN under another scale -8 (the median of a NaN and
+// the bounds is the lower one), as the division with its clamp did.
 __device__ __forceinline__ uint32_t codes8(const float* x, float rs) {
   uint32_t acc = 0;
 #pragma unroll
@@ -78,7 +80,7 @@ __device__ __forceinline__ uint32_t codes8(const float* x, float rs) {
     acc = (acc << 4) + __float_as_uint(c);
   }
   constexpr uint32_t kBias = 0x4B400000u + (0x4B400000u << 4) + (0x4B400000u << 8);   // higher terms vanish mod 2^32
-  return (acc - kBias + 0x88888888u) ^ 0x88888888u;
+  return rs != 0.0f ? (acc - kBias + 0x88888888u) ^ 0x88888888u : 0u;
 }
 
 // Max over the LANES (4, 8 or 16) lanes of an aligned group, on the bit

@@ -72,6 +72,32 @@ def test_scales_at_the_ends_of_fp16(dtype, scale):
     assert np.array_equal(stats.cpu().numpy().view(np.uint64).reshape(2, 128), want.reshape(2, 128))
 
 
+def test_nan_and_infinity():
+    """A NaN is left out of its group's scale; its code is -8, and 0 where the scale is 0 (a group of NaN
+    and zeros).  An infinity saturates the scale and takes the outermost code."""
+    key = torch.zeros((1, 1, 64, 128), dtype=torch.bfloat16, device=DEV)
+    key[0, 0, :, 3] = float("nan")       # group 0: NaN and zeros
+    key[0, 0, :, 40] = float("nan")      # group 1: NaN among ordinary values
+    key[0, 0, :, 41:48] = 7.0
+    key[0, 0, :, 70] = float("inf")      # group 2
+    key[0, 0, :, 71] = -float("inf")
+    packed, scales = K.int4_pack_k(key, 32)
+    codes = torch.stack([packed[0, 0, :64] & 15, packed[0, 0, :64] >> 4], dim=-1).view(64, 128).cpu()
+    codes = torch.where(codes > 7, codes.int() - 16, codes.int())
+    want = torch.zeros(128, dtype=torch.int32)
+    want[40], want[41:48], want[70], want[71] = -8, 7, 7, -8
+    assert torch.equal(codes, want.expand(64, 128))
+    assert scales[0, 0, 0].tolist() == [0.0, 1.0, 65504.0, 0.0]
+    chan = torch.arange(16, dtype=torch.int32, device=DEV).view(1, 1, 16)   # the first group's channels only
+    for kk in (key, unaligned(key)):
+        slab = torch.full((1, 1, K.round_capacity(64), 8), 7, dtype=torch.uint8, device=DEV)
+        ss = torch.zeros(slab.shape[:3], dtype=torch.float16, device=DEV)
+        K.build_slab(kk, chan, slab=slab, slab_scales=ss)
+        stored = O.swizzle_slab(np.zeros((1, 64, 8), np.uint8), K.round_capacity(64)).reshape(-1)
+        mask = O.swizzle_slab(np.full((1, 64, 8), 255, np.uint8), K.round_capacity(64)).reshape(-1) != 0
+        assert np.array_equal(slab.cpu().numpy().reshape(-1)[mask], stored[mask])
+
+
 def test_statistic_without_workspace():
     key = make(2, 4, 3000, 128, torch.bfloat16, 9)
     packed, scales = K.int4_pack_k(key, 32)
