@@ -261,8 +261,10 @@ int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_heads, int6
 /* The same with a state the caller keeps (optional; qkv_topk_state_bytes(rows,
  * tokens, k) bytes, 16-byte aligned, 0 where the sizes use none): zero-filled
  * once, left zero by every completed call, so that no launch clears the row
- * histograms.  Calls sharing a state must not overlap in time and must have
- * the same number of rows. */
+ * histograms (a call that fails after counting clears it).  Calls sharing a
+ * state must not overlap in time; after two that did it has to be zero-filled
+ * again.  A call on a state that is not zero may select fewer than k keys, its
+ * remaining indices -1, and never one twice or out of the row. */
 int64_t qkv_topk_state_bytes(int64_t rows, int64_t n, int64_t k);
 int qkv_int4_decode_topk_state(const void* query, int64_t batch, int64_t q_heads, int64_t kv_heads,
                                int64_t head_dim, const int32_t* chan_idx, int64_t selected, const uint8_t* slab,

@@ -478,7 +478,7 @@ __global__ __launch_bounds__(64 * win_waves(S)) void decode_scores_win_kernel(
                                   1, kStageChunk, scores, tokens, nullptr, nullptr, qscale_out, blockIdx.y,
                                   blockIdx.x, h);
   __syncthreads();
-  if (row_hist) {   // uniform: the row histogram of a large k instead
+  if (row_hist) {   // uniform: counted into the row's histogram instead
     flush_row_hist<NT>(h, row_hist + blockIdx.y * hist_stride);
     return;
   }
@@ -783,6 +783,7 @@ int64_t topk_hist_stride();
 int topk_big_clear(int64_t rows, int64_t n, void* workspace, hipStream_t st, int** hist, int64_t* stride);
 int topk_big_finish(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
                     void* workspace, int* state, hipStream_t st);
+void topk_state_clear(int64_t rows, int* state, hipStream_t st);
 }  // namespace qkv
 
 QKV_EXPORT int qkv_int4_decode_topk(const void* query, int64_t batch, int64_t q_heads, int64_t kv_heads,
@@ -868,8 +869,9 @@ QKV_EXPORT int qkv_int4_decode_topk_state(const void* query, int64_t batch, int6
     case 128: rc = with_f(std::integral_constant<int, 128>{}); break;
     default: return fail(QKV_ERR_UNSUPPORTED, "%s: selected channel count %lld not built", what, (long long)selected);
   }
-  if (rc) return rc;
-  if (row_hist)
-    return topk_big_finish(scores, rows, tokens, tokens, k, out, workspace, kept ? hist : nullptr, st);
+  if (!rc && row_hist)
+    rc = topk_big_finish(scores, rows, tokens, tokens, k, out, workspace, kept ? hist : nullptr, st);
+  if (rc && kept) topk_state_clear(rows, hist, st);   // the scores may have been counted
+  if (rc || row_hist) return rc;
   return topk_filtered(scores, rows, tokens, tokens, k, out, workspace, st, true);
 }

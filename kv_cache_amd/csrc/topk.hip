@@ -1332,7 +1332,7 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
   __shared__ typename WS::Shared sh;
   __shared__ int wave_cnt[16];
   __shared__ int pre[kBigSlices + 1];
-  __shared__ int last_sh, over_sh;
+  __shared__ int last_sh, over_sh, have_sh;
   const int row = blockIdx.x / slices, s = blockIdx.x - row * slices;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int* hrow = hist + static_cast<int64_t>(row) * kBigStride;
@@ -1405,11 +1405,13 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
     const int c = tid < slices ? ld_coherent(state + tid) : 0;
     const uint64_t over = __ballot(c > cap);
     const int inc = wave_incl_scan_dpp(min(c, cap));
+    const int all = wave_incl_scan_dpp(c);
     if (tid < slices) pre[tid + 1] = inc;
     if (tid == 0) {
       pre[0] = 0;
       over_sh = over != 0;
     }
+    if (tid == 63) have_sh = all;
   }
   for (int j = tid; j < n_words; j += 1024)
     fw[j] = __hip_atomic_load(wrow + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1432,7 +1434,10 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
     *reinterpret_cast<int4*>(hist + static_cast<int64_t>(row) * kBigStride + 4 * tid) = make_int4(0, 0, 0, 0);
     if (tid < kBigState) state[tid] = 0;
   }
-  if (over_sh)   // uniform
+  // The bin holds at least `rank` keys; a histogram that was not zero when the
+  // row was counted may say otherwise, and then none is taken.
+  if (have_sh < rank) {   // uniform
+  } else if (over_sh)
     bin_taken_stream(&sh, n, rank, bin, n, fw, [&](int p, float& x, int& pos) {
       x = vrow[p];
       pos = p;
@@ -1453,10 +1458,14 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
   const int incl = wave_incl_scan_dpp(cnt);
   if (lane == 63) wave_cnt[wave] = incl;
   __syncthreads();
-  int p = incl - cnt;
+  int p = incl - cnt, taken = 0;
 #pragma unroll
-  for (int w = 0; w < 16; ++w) p += w < wave ? wave_cnt[w] : 0;
+  for (int w = 0; w < 16; ++w) {
+    p += w < wave ? wave_cnt[w] : 0;
+    taken += wave_cnt[w];
+  }
   int32_t* orow = out + static_cast<int64_t>(row) * k;
+  for (int at = taken + tid; at < k; at += 1024) orow[at] = -1;   // (not reached from a zero histogram)
   for (int j = 0; j < wpt; ++j) {
     const int w = tid * wpt + j;
     if (w >= n_words) break;
@@ -1673,6 +1682,12 @@ int topk_big_clear(int64_t rows, int64_t n, void* workspace, hipStream_t st, int
   *hist = w.hist;
   *stride = kBigStride;
   return check_launch("qkv_topk_ws");
+}
+
+// Zeroes a state the caller keeps, after a call that could not finish.
+void topk_state_clear(int64_t rows, int* state, hipStream_t st) {
+  const int64_t n4 = rows * kBigStride / 4;
+  topk_clear_kernel<<<static_cast<unsigned>(cdiv(n4, 256)), 256, 0, st>>>(reinterpret_cast<int4*>(state), n4);
 }
 
 // state: the zero-filled histogram and state to use (and to leave zero)

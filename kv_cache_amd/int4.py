@@ -219,6 +219,8 @@ def decode_topk(query: torch.Tensor, chan_idx: torch.Tensor, slab: torch.Tensor,
              and scores.size(-1) == t, "scores must be contiguous float32 [B,Hkv,tokens]")
     if out is None:
         out = torch.empty((b, hkv, int(k)), dtype=torch.int32, device=q.device)
+    _require(state is None or (state.device == q.device and state.is_contiguous()),
+             "state must be contiguous on the query's device")
     need = lib.qkv_topk_workspace_bytes(b * hkv, t, int(k))
     _require(need >= 0, f"bad top-k sizes tokens={t} k={k}")
     if need > 0 and (workspace is None or workspace.numel() * 4 < need):
@@ -228,14 +230,16 @@ def decode_topk(query: torch.Tensor, chan_idx: torch.Tensor, slab: torch.Tensor,
             q.data_ptr(), b, hq, hkv, d, chan_idx.data_ptr(), s, slab.data_ptr(), slab_scales.data_ptr(), cap, t,
             int(k), scores.data_ptr(), out.data_ptr(), _lib.ptr(workspace),
             0 if workspace is None else workspace.numel() * 4, _lib.ptr(state),
-            0 if state is None else state.numel() * 4, code, _lib.stream_of(q)))
+            0 if state is None else state.numel() * state.element_size(), code, _lib.stream_of(q)))
     return out
 
 
 def topk_state(rows: int, n: int, k: int, device) -> torch.Tensor | None:
     """Zero-filled state for ``decode_topk`` calls of these sizes (None where
     they use none); every completed call leaves it zero.  Calls sharing a
-    state must not overlap in time."""
+    state must not overlap in time: after two that did, ``zero_()`` it (a call
+    on a state that is not zero may select too few keys, the rest of its
+    indices -1)."""
     need = _lib.load().qkv_topk_state_bytes(int(rows), int(n), int(k))
     _require(need >= 0, f"bad top-k sizes rows={rows} n={n} k={k}")
     return torch.zeros(need // 4, dtype=torch.int32, device=device) if need else None

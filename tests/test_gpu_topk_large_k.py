@@ -105,6 +105,43 @@ def test_kept_state_returns_to_zero(tokens, k):
         K.decode_topk(q, cache.chan_idx, cache.slab, cache.slab_scales, tokens, k, workspace=ws, state=state[:64])
 
 
+@pytest.mark.parametrize("tokens,k", [(5000, 300), (40000, 1024), (131072, 4000)])
+def test_state_left_with_counts(tokens, k):
+    """Counts left in a state (here k keys of the highest bin, which the row does not hold): no index
+    is stale, and the call leaves the state zero, so that the next one is exact."""
+    g = torch.Generator().manual_seed(k)
+    key = torch.randn((1, 4, tokens, 128), generator=g).to(torch.bfloat16).to(DEV)
+    cache = K.Int4KCache.from_prefill(key, 32, 32)
+    q = torch.randn((1, 8, 128), generator=g).to(torch.bfloat16).to(DEV)
+    state = K.topk_state(4, tokens, k, DEV)
+    stride = 4096 + 64 + 8
+    state[4095 : 4 * stride : stride] = k
+    scores = torch.empty((1, 4, tokens), device=DEV)
+    out = torch.full((1, 4, k), 7, dtype=torch.int32, device=DEV)
+    K.decode_topk(q, cache.chan_idx, cache.slab, cache.slab_scales, tokens, k, scores=scores, out=out, state=state)
+    assert bool((out == -1).all()) and int(state.abs().sum()) == 0
+    K.decode_topk(q, cache.chan_idx, cache.slab, cache.slab_scales, tokens, k, scores=scores, out=out, state=state)
+    assert np.array_equal(out.cpu().numpy().reshape(4, k), want(scores.cpu().view(4, tokens), k))
+
+
+def test_state_arguments():
+    key = torch.randn((1, 2, 5000, 128), generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(DEV)
+    cache = K.Int4KCache.from_prefill(key, 32, 32)
+    q = torch.randn((1, 4, 128), generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).to(DEV)
+    words = K.topk_state(2, 5000, 64, DEV).numel()
+
+    def call(state):
+        return K.decode_topk(q, cache.chan_idx, cache.slab, cache.slab_scales, 5000, 64, state=state)
+
+    with pytest.raises(RuntimeError, match="contiguous"):
+        call(torch.zeros(1, dtype=torch.int32, device=DEV).expand(words))
+    with pytest.raises(RuntimeError, match="device"):
+        call(torch.zeros(words, dtype=torch.int32))
+    with pytest.raises(RuntimeError, match="state needs"):   # bytes, not elements
+        call(torch.zeros(words, dtype=torch.uint8, device=DEV))
+    assert torch.equal(call(torch.zeros(words, device=DEV)), call(None))
+
+
 @pytest.mark.parametrize("n,k", [(5000, 64), (9000, 1000), (131072, 1024), (196609, 500)])
 def test_smaller_workspaces_take_the_chunk_lists(n, k):
     """Workspaces sized for the chunk lists (their size does not depend on the row histogram) are still accepted."""
