@@ -1186,7 +1186,8 @@ __global__ __launch_bounds__(1024) void topk_fused_kernel(const float* __restric
 // the row's position word s * 16 * J + w * J + i) finds the boundary bin from
 // that histogram, writes its words with the keys above the bin set, and lists
 // its keys inside the bin in position order (up to `cap`; their true count
-// goes to state[s]).  The row's last slice to take its ticket resolves the
+// goes to state[s]); a slice with more of them than that lists its largest
+// `rank` only, where that is fewer.  The row's last slice to take its ticket resolves the
 // bin (from the list in registers, in memory, or, where a slice's list
 // overflowed, from the row itself), sets the taken positions in an LDS bitset
 // of the row and writes the positions in ascending order.  Slices store
@@ -1198,11 +1199,16 @@ __global__ __launch_bounds__(1024) void topk_fused_kernel(const float* __restric
 // slice's two passes and its output): 11.6 us at 32 rows x 20010 keys with k =
 // 1001 (13.7 in topk_fused_kernel), 12.2 at 8 rows x 131072 with k = 1024
 // (17.4) and at 8 x 131071 with k = 6554 (222 us, one workgroup per row).
+// Rows with a large share of their keys in one bin (1/8 octave) take longer: 8
+// rows x 131072 keys 100 + 0.5 z, k = 64 and 1000, 31 and 113 us with the two
+// launches before (163 where the last slice reads the row; chunk lists 35 and
+// 62), equal keys 36 and 126 (336; chunk lists 32 and 60).
 // ---------------------------------------------------------------------------
 constexpr int64_t kBigMax = 192 * 1024;    // positions whose bitset fits beside the selection in 64 KB of LDS
 constexpr int kBigSlices = 64;             // slices per row, one lane of a wave each
 constexpr int kBigState = kBigSlices + 8;  // ints per row: the slices' counts, then the ticket
 constexpr int kBigStride = kHistBins + kBigState;   // ints per row of histogram and state
+constexpr int kBigListed = 8 * 1024;       // keys of the boundary bin resolved in registers
 
 __global__ __launch_bounds__(256) void topk_clear_kernel(int4* __restrict__ p, int64_t n) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -1257,9 +1263,12 @@ __device__ void bin_taken(void* raw, int m, int rank, int bin, int n, uint64_t* 
 }
 
 // The same for keys too many for registers, read anew on every pass; keys
-// outside the bin may be among them.
+// outside the bin may be among them.  A thread adds equal digits that follow
+// one another in one atomic, or equal keys would take one address in turn.
+// (Four loads in flight a thread are 10% faster here, and cost the common path
+// of topk_slices_kernel 1 to 4% through its registers.)
 template <typename Get>
-__device__ void bin_taken_stream(void* raw, int m, int rank, int bin, int n, uint64_t* fw, Get&& get) {
+__device__ __forceinline__ void bin_taken_stream(void* raw, int m, int rank, int bin, int n, uint64_t* fw, Get&& get) {
   using WS = WideSelect<1, false>;
   auto& sh = *static_cast<typename WS::Shared*>(raw);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1274,13 +1283,23 @@ __device__ void bin_taken_stream(void* raw, int m, int rank, int bin, int n, uin
   while (remaining > 0) {   // uniform
     const int shift = remaining > WS::RB ? remaining - WS::RB : 0;
     const uint32_t dmask = (1u << (remaining - shift)) - 1u;
+    uint32_t digit = 0;
+    int run = 0;
+#pragma unroll 1
     for (int p = tid; p < m; p += 1024) {
       float v;
       int at;
       get(p, v, at);
-      const uint32_t u = f32_sortable(v);
-      if ((u & mask) == prefix) atomicAdd(&sh.hist[buf][(u >> shift) & dmask], 1);
+      const uint32_t u = f32_sortable(v), d = (u >> shift) & dmask;
+      if ((u & mask) != prefix) continue;
+      if (d != digit && run) {
+        atomicAdd(&sh.hist[buf][digit], run);
+        run = 0;
+      }
+      digit = d;
+      ++run;
     }
+    if (run) atomicAdd(&sh.hist[buf][digit], run);
     __syncthreads();
     int b, krl, whole;
     ws.boundary(sh, sh.hist[buf], sh.hist[buf ^ 1], b, krl, whole);
@@ -1294,6 +1313,7 @@ __device__ void bin_taken_stream(void* raw, int m, int rank, int bin, int n, uin
   // prefix: theta; equal keys are taken while fewer than kr came before
   const int kr = ws.kr;
   int eq_seen = 0;   // equal keys in the earlier rounds (uniform)
+#pragma unroll 1
   for (int p0 = 0; p0 < m; p0 += 1024) {   // uniform
     const int p = p0 + tid;
     float v = 0.0f;
@@ -1332,7 +1352,7 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
   __shared__ typename WS::Shared sh;
   __shared__ int wave_cnt[16];
   __shared__ int pre[kBigSlices + 1];
-  __shared__ int last_sh, over_sh, have_sh;
+  __shared__ int last_sh, over_sh;
   const int row = blockIdx.x / slices, s = blockIdx.x - row * slices;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int* hrow = hist + static_cast<int64_t>(row) * kBigStride;
@@ -1372,20 +1392,58 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
     at += w < wave ? wave_cnt[w] : 0;
     total += wave_cnt[w];
   }
-  if (tid == 0) st_coherent(state + s, total);
-  if (wtot) {   // uniform per wave
-    const int64_t base = (static_cast<int64_t>(row) * slices + s) * cap;
+  const int64_t lists = (static_cast<int64_t>(row) * slices + s) * cap;
+  if (__builtin_expect(total > cap && slices > 2 && rank <= cap, 0)) {   // uniform
+    // More keys of the bin than the list holds, fewer of them wanted: only the
+    // slice's own first `rank` can be among them, so it lists those.  (Rows of
+    // one or two slices are as fast read by the last one.)
+    const int base = s * 1024 * J, word0 = s * 16 * J, words_here = min(16 * J, n_words - word0);
+    for (int j = tid; j < words_here; j += 1024) fw[word0 + j] = 0;
+    __syncthreads();
+    bin_taken_stream(&sh, min(1024 * J, n - base), rank, bin, n, fw, [&](int p, float& x, int& pos) {
+      x = vrow[base + p];
+      pos = base + p;
+    });
+    const int own = lane < J && w0 + lane < n_words ? __popcll(fw[w0 + lane]) : 0;   // lane i: the wave's word i
+    const int incl = wave_incl_scan_dpp(own);
+    if (lane == 63) wave_cnt[wave] = incl;
+    __syncthreads();
+    int first = 0, listed = 0;
 #pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      first += w < wave ? wave_cnt[w] : 0;
+      listed += wave_cnt[w];
+    }
+    if (tid == 0) st_coherent(state + s, listed);
+#pragma unroll 2
     for (int i = 0; i < J; ++i) {
-      if ((bal[i] >> lane) & 1ull) {
-        const int e = at + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-                               static_cast<uint32_t>(bal[i] >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bal[i]), 0)));
+      const uint64_t x = w0 + i < n_words ? fw[w0 + i] : 0ull;
+      const int word_at = first + __builtin_amdgcn_readlane(incl - own, i);
+      if ((x >> lane) & 1ull) {
+        const int e = word_at + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                                    static_cast<uint32_t>(x >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(x), 0)));
+        const int pos = 64 * (w0 + i) + lane;
         if (e < cap) {
-          st_coherent(list_val + base + e, v[i]);
-          st_coherent(list_pos + base + e, 64 * (w0 + i) + lane);
+          st_coherent(list_val + lists + e, vrow[pos]);
+          st_coherent(list_pos + lists + e, pos);
         }
       }
-      at += __popcll(bal[i]);
+    }
+  } else {
+    if (tid == 0) st_coherent(state + s, total);
+    if (wtot) {   // uniform per wave
+#pragma unroll
+      for (int i = 0; i < J; ++i) {
+        if ((bal[i] >> lane) & 1ull) {
+          const int e = at + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                                 static_cast<uint32_t>(bal[i] >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bal[i]), 0)));
+          if (e < cap) {
+            st_coherent(list_val + lists + e, v[i]);
+            st_coherent(list_pos + lists + e, 64 * (w0 + i) + lane);
+          }
+        }
+        at += __popcll(bal[i]);
+      }
     }
   }
   // Every word, count and list store of this workgroup has completed before its ticket.
@@ -1405,13 +1463,11 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
     const int c = tid < slices ? ld_coherent(state + tid) : 0;
     const uint64_t over = __ballot(c > cap);
     const int inc = wave_incl_scan_dpp(min(c, cap));
-    const int all = wave_incl_scan_dpp(c);
     if (tid < slices) pre[tid + 1] = inc;
     if (tid == 0) {
       pre[0] = 0;
       over_sh = over != 0;
     }
-    if (tid == 63) have_sh = all;
   }
   for (int j = tid; j < n_words; j += 1024)
     fw[j] = __hip_atomic_load(wrow + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1436,17 +1492,21 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
   }
   // The bin holds at least `rank` keys; a histogram that was not zero when the
   // row was counted may say otherwise, and then none is taken.
-  if (have_sh < rank) {   // uniform
-  } else if (over_sh)
-    bin_taken_stream(&sh, n, rank, bin, n, fw, [&](int p, float& x, int& pos) {
-      x = vrow[p];
-      pos = p;
-    });
-  else if (m <= 1024) bin_taken<1>(&sh, m, rank, bin, n, fw, from_list);
+  const bool over = over_sh;
+  if (__builtin_expect(over || m > kBigListed || m < rank, 0)) {   // uniform
+    if (over || m >= rank)
+      bin_taken_stream(&sh, over ? n : m, rank, bin, n, fw, [&](int p, float& x, int& pos) {
+        if (over) {
+          x = vrow[p];
+          pos = p;
+        } else {
+          from_list(p, x, pos);
+        }
+      });
+  } else if (m <= 1024) bin_taken<1>(&sh, m, rank, bin, n, fw, from_list);
   else if (m <= 2 * 1024) bin_taken<2>(&sh, m, rank, bin, n, fw, from_list);
   else if (m <= 4 * 1024) bin_taken<4>(&sh, m, rank, bin, n, fw, from_list);
-  else if (m <= 8 * 1024) bin_taken<8>(&sh, m, rank, bin, n, fw, from_list);
-  else bin_taken_stream(&sh, m, rank, bin, n, fw, from_list);
+  else bin_taken<8>(&sh, m, rank, bin, n, fw, from_list);
   __syncthreads();
   // the taken positions, ascending: consecutive words per thread
   const int wpt = (n_words + 1023) / 1024;
@@ -1511,7 +1571,7 @@ int big_j(int64_t rows, int64_t n) {
 
 // List entries a slice of 1024 * j keys may hold (a 12-bit bin of normal
 // scores holds some 2% of the keys).
-int64_t big_cap(int j) { return 1024 * j / 8; }
+int64_t big_cap(int j) { return 1024 * j / 4; }
 
 struct BigWs {
   int* hist;

@@ -1,5 +1,6 @@
-"""Top-k with k past the chunk lists on long rows (row histogram and slices): every tie pattern, list
-lengths in registers, in memory and overflowing, and the decode call that counts as it scores."""
+"""Top-k of long rows by row histogram and slices: every tie pattern, boundary bins that hold few keys,
+most of them or all, lists in registers and in memory, and the decode call that counts as it scores;
+and the calls that take one workgroup per row or the chunk lists instead."""
 
 import numpy as np
 import pytest
@@ -36,8 +37,6 @@ def want(vals, k):
 @pytest.mark.parametrize("share", [0.0, 0.1, 0.5, 1.0])
 @pytest.mark.parametrize("copies", [1, 20])   # 6 or 120 rows: other keys per thread
 def test_large_k_equals_stable_sort(n, share, copies):
-    if copies > 1 and n > 65536:
-        pytest.skip("the same slices as the shorter rows")
     k = max(1025, min(n, int(share * n)))
     vals = rows_of(n, n + copies)
     assert _lib.load().qkv_topk_workspace_bytes(6, n, k) > 0
@@ -50,6 +49,24 @@ def test_large_k_equals_stable_sort(n, share, copies):
         assert (got == got[:1]).all()
 
 
+@pytest.mark.parametrize("n", [4097, 9001, 20003, 131072, 196608])
+@pytest.mark.parametrize("k", [1, 300, 513, 1024])
+@pytest.mark.parametrize("copies", [1, 20])
+def test_boundary_bins_of_many_keys(n, k, copies):
+    """Slices that hold more keys of the boundary bin than are wanted of it list only their first ones."""
+    few = torch.full((2, n), -float("inf"))    # k past the finite keys: the rest is -inf, lowest index first
+    few[0, 5::(n // 40)] = 1.0
+    few[1, : min(n, 900)] = torch.randn(min(n, 900), generator=torch.Generator().manual_seed(k))
+    narrow = 100.0 + 0.5 * torch.randn((2, n), generator=torch.Generator().manual_seed(n))
+    narrow[1, n // 2 :] = 100.25               # equal keys behind distinct ones of the same bin
+    vals = torch.cat([rows_of(n, n + k), few, narrow])
+    rows = vals.size(0)
+    ws = K.topk_workspace(rows * copies, n, k, DEV)
+    got = K.block_topk(vals.repeat(copies, 1).to(DEV), k, workspace=ws).cpu().numpy().reshape(copies, rows, k)
+    assert np.array_equal(got[0], want(vals, k))
+    assert (got == got[:1]).all()
+
+
 def test_calls_without_the_larger_workspace_still_run():
     lib = _lib.load()
     vals = rows_of(9000, 4).to(DEV)
@@ -58,7 +75,7 @@ def test_calls_without_the_larger_workspace_still_run():
     assert np.array_equal(out.cpu().numpy(), want(vals.cpu(), 2000))
 
 
-@pytest.mark.parametrize("tokens,k,selected", [(5000, 1200, 16), (20011, 2002, 32), (70001, 7001, 64), (8192, 8192, 128)])
+@pytest.mark.parametrize("tokens,k,selected", [(5000, 1024, 16), (5000, 1200, 16), (20011, 2002, 32), (70001, 7001, 64), (8192, 8192, 128)])
 def test_decode_topk_counts_as_it_scores(tokens, k, selected):
     g = torch.Generator().manual_seed(tokens)
     key = torch.randn((2, 3, tokens, 128), generator=g).to(torch.bfloat16).to(DEV)
