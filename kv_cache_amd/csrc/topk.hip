@@ -1826,10 +1826,20 @@ int64_t topk_least_bytes(int64_t rows, int64_t n, int64_t k) {
   return big(n) && rows <= 65535 ? std::min(lists, big_ws(nullptr, rows, n).bytes) : lists;
 }
 
-// Whether a call takes the row-histogram path: its sizes, and a workspace that holds it.
-bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes) {
-  return rows > 0 && rows <= 65535 && k >= 1 && k <= n && big(n) && workspace && aligned(workspace, 16) &&
-         bytes >= big_ws(nullptr, rows, n).bytes;
+// Whether a call takes the row-histogram path: its sizes, and a workspace that
+// holds it.  kept: a scoring launch counts the keys into a state that needs no
+// clearing.
+// Where the other paths are faster, us of the row histogram and of the other:
+//   k past the chunk lists, one workgroup per row as long as it holds the row
+//   in registers and LDS: 8 rows x 4100 15.5 and 9.2, x 8192 15.1 and 11.7,
+//   x 12288 15.1 and 13.6 (512 rows 46.9 and 19.5), x 12300 15.3 and 19.6;
+//   kept, with the scores, 8 rows x 6000 15.7 and 14.3, x 12288 15.8 and 19.0
+//   (k = 6144 18.6 and 19.2), 256 rows x 9000 31.5 and 25.8.
+bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes, bool kept) {
+  if (rows <= 0 || rows > 65535 || k < 1 || k > n || !big(n) || !workspace || !aligned(workspace, 16)) return false;
+  if (bytes < big_ws(nullptr, rows, n).bytes) return false;
+  if (k > kStageMaxK) return n > kLdsKeys || (kept && n > 2 * kStageChunk && rows <= 128 && k <= n / 4);
+  return true;
 }
 }  // namespace qkv
 
@@ -1855,7 +1865,7 @@ QKV_EXPORT int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k) 
 
 QKV_EXPORT int qkv_topk_ws(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
                            void* workspace, int64_t workspace_bytes, void* stream) {
-  const bool row_hist = topk_takes_row_hist(rows, n, k, workspace, workspace_bytes);
+  const bool row_hist = topk_takes_row_hist(rows, n, k, workspace, workspace_bytes, false);
   if (!staged(n, k) && !row_hist) return qkv_topk(values, rows, n, ld, k, out, stream);
   if (!values || !out || !workspace) return fail(QKV_ERR_INVALID, "qkv_topk_ws: null pointer");
   if (rows <= 0 || rows > 65535 || ld < n || n >= (int64_t(1) << 31))

@@ -67,6 +67,24 @@ def test_boundary_bins_of_many_keys(n, k, copies):
     assert (got == got[:1]).all()
 
 
+@pytest.mark.parametrize("batch,tokens,k", [(33, 33000, 700), (33, 4200, 64), (17, 9000, 1100), (4, 12288, 1500),
+                                            (4, 12289, 6000), (1, 8192, 1025)])
+def test_decode_topk_by_rows_and_k(batch, tokens, k):
+    """Both sides of the lines between the row histogram, the chunk lists and one workgroup per row, with
+    and without a kept state, which stays zero whichever is taken."""
+    g = torch.Generator(device=DEV).manual_seed(tokens)
+    key = torch.randn((batch, 8, tokens, 128), generator=g, device=DEV).to(torch.bfloat16)
+    q = torch.randn((batch, 16, 128), generator=g, device=DEV).to(torch.bfloat16)
+    cache = K.Int4KCache.from_prefill(key, 32, 16)
+    scores = K.decode_scores(q, cache.chan_idx, cache.slab, cache.slab_scales, tokens, 1)
+    order = torch.sort(scores.view(-1, tokens), dim=1, descending=True, stable=True).indices[:, :k]
+    state = K.topk_state(batch * 8, tokens, k, DEV)
+    for st in (None, state, state):
+        got = K.decode_topk(q, cache.chan_idx, cache.slab, cache.slab_scales, tokens, k, state=st)
+        assert torch.equal(got.view(-1, k), order.sort(dim=1).values.int())
+    assert not state.any()
+
+
 def test_calls_without_the_larger_workspace_still_run():
     lib = _lib.load()
     vals = rows_of(9000, 4).to(DEV)
