@@ -778,7 +778,8 @@ namespace qkv {
 int topk_filtered(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
                   void* workspace, hipStream_t st, bool given);
 bool topk_takes_windows(int64_t n, int64_t k);
-bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes, bool kept);
+bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes, bool counted,
+                         bool kept);
 int64_t topk_hist_stride();
 int topk_big_clear(int64_t rows, int64_t n, void* workspace, hipStream_t st, int** hist, int64_t* stride);
 int topk_big_finish(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
@@ -821,7 +822,7 @@ QKV_EXPORT int qkv_int4_decode_topk_state(const void* query, int64_t batch, int6
     return fail(QKV_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
                 (long long)workspace_bytes);
   if (need > 0 && !aligned(workspace, 16)) return fail(QKV_ERR_INVALID, "%s: workspace must be 16-byte aligned", what);
-  const bool row_hist = topk_takes_row_hist(rows, tokens, k, workspace, workspace_bytes, state != nullptr);
+  const bool row_hist = topk_takes_row_hist(rows, tokens, k, workspace, workspace_bytes, true, state != nullptr);
   if (!(topk_takes_windows(tokens, k) || row_hist) || rows > 65535) {   // the scores, then qkv_topk_ws as it stands
     if (int rc = qkv_int4_decode_scores(query, batch, q_heads, kv_heads, head_dim, chan_idx, selected, slab,
                                         slab_scales, capacity, tokens, 1, scores, nullptr, nullptr, nullptr, dtype,

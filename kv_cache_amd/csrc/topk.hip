@@ -1562,10 +1562,12 @@ bool filtered(int64_t n, int64_t k) {
 bool big(int64_t n) { return n > kStageChunk && n <= kBigMax; }
 
 // Keys per thread of a slice: the fewest that keep the grid within 256
-// workgroups (one per CU) and a row within kBigSlices slices.
+// workgroups (one per CU) and a row within kBigSlices slices, and no more
+// than one slice a row takes.
 int big_j(int64_t rows, int64_t n) {
   int j = 4;
-  while (j < 32 && (rows * cdiv(n, int64_t(1024) * j) > 256 || cdiv(n, int64_t(1024) * j) > kBigSlices)) j *= 2;
+  auto slices = [&] { return cdiv(n, int64_t(1024) * j); };
+  while (j < 32 && slices() > 1 && (rows * slices() > 256 || slices() > kBigSlices)) j *= 2;
   return j;
 }
 
@@ -1827,19 +1829,29 @@ int64_t topk_least_bytes(int64_t rows, int64_t n, int64_t k) {
 }
 
 // Whether a call takes the row-histogram path: its sizes, and a workspace that
-// holds it.  kept: a scoring launch counts the keys into a state that needs no
-// clearing.
+// holds it.  counted: a scoring launch counts the keys (and could build the
+// chunk lists' windows as well); kept: into a state that needs no clearing.
 // Where the other paths are faster, us of the row histogram and of the other:
 //   k past the chunk lists, one workgroup per row as long as it holds the row
 //   in registers and LDS: 8 rows x 4100 15.5 and 9.2, x 8192 15.1 and 11.7,
 //   x 12288 15.1 and 13.6 (512 rows 46.9 and 19.5), x 12300 15.3 and 19.6;
 //   kept, with the scores, 8 rows x 6000 15.7 and 14.3, x 12288 15.8 and 19.0
 //   (k = 6144 18.6 and 19.2), 256 rows x 9000 31.5 and 25.8.
-bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes, bool kept) {
+//   More than 256 rows, scores counted, whose last slice is mostly past the
+//   row: 264 rows x 33000 90 and 79, 1024 x 66000 465 and 437; with 1.23 times
+//   the row in slices 264 x 80000 140 and 150.
+//   512 rows and more past the lists one workgroup merges, not counted (the
+//   stages read the row once): 512 rows x 196608, k = 1000, 338 and 300 (300
+//   rows x 160000 157 and 169).
+bool topk_takes_row_hist(int64_t rows, int64_t n, int64_t k, const void* workspace, int64_t bytes, bool counted,
+                         bool kept) {
   if (rows <= 0 || rows > 65535 || k < 1 || k > n || !big(n) || !workspace || !aligned(workspace, 16)) return false;
   if (bytes < big_ws(nullptr, rows, n).bytes) return false;
   if (k > kStageMaxK) return n > kLdsKeys || (kept && n > 2 * kStageChunk && rows <= 128 && k <= n / 4);
-  return true;
+  if (rows <= 256 || bytes < staged_bytes(rows, n, k)) return true;
+  if (!counted) return rows < 512 || filtered(n, k);
+  const int64_t slice = int64_t(1024) * big_j(rows, n);
+  return !filtered(n, k) || 4 * cdiv(n, slice) * slice <= 5 * n;
 }
 }  // namespace qkv
 
@@ -1857,15 +1869,16 @@ QKV_EXPORT int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k) 
   if (rows <= 0 || n <= 0 || k < 1 || k > n) return -1;
   if (rows > 65535 || n <= kStageChunk) return staged_bytes(rows, n, k);
   const int64_t hist = big_ws(nullptr, rows, std::min(n, kBigMax)).bytes;
-  if (n <= kBigMax) return hist;
   const int64_t kl = std::min<int64_t>(k, kStageMaxK);
+  if (n <= kBigMax)   // (from 512 rows the stages past kFilterMaxLists, too)
+    return rows >= 512 && n * kStageMaxK > kFilterMaxLists * kStageChunk ? std::max(hist, staged_bytes(rows, n, kl)) : hist;
   const int64_t windows_end = std::min<int64_t>(n, kFilterMaxChunks * kStageChunk);
   return std::max({hist, staged_bytes(rows, n, kl), staged_bytes(rows, windows_end, kl)});
 }
 
 QKV_EXPORT int qkv_topk_ws(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k, int32_t* out,
                            void* workspace, int64_t workspace_bytes, void* stream) {
-  const bool row_hist = topk_takes_row_hist(rows, n, k, workspace, workspace_bytes, false);
+  const bool row_hist = topk_takes_row_hist(rows, n, k, workspace, workspace_bytes, false, false);
   if (!staged(n, k) && !row_hist) return qkv_topk(values, rows, n, ld, k, out, stream);
   if (!values || !out || !workspace) return fail(QKV_ERR_INVALID, "qkv_topk_ws: null pointer");
   if (rows <= 0 || rows > 65535 || ld < n || n >= (int64_t(1) << 31))

@@ -67,6 +67,19 @@ def test_boundary_bins_of_many_keys(n, k, copies):
     assert (got == got[:1]).all()
 
 
+@pytest.mark.parametrize("rows,n,k", [(257, 4097, 700), (300, 20003, 64), (257, 33000, 1000), (512, 135169, 1000), (257, 135169, 1000),
+                                      (513, 8193, 1100), (257, 12289, 1100)])
+def test_more_rows_than_workgroups_at_once(rows, n, k):
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    vals = torch.randn((rows, n), generator=g, device=DEV)
+    vals[rows // 2] = 3.0
+    got = K.block_topk(vals, k)
+    some = [0, 1, rows // 2, 255, 256, rows - 1]
+    assert np.array_equal(got[some].cpu().numpy(), want(vals[some].cpu(), k))
+    order = torch.sort(vals, dim=1, descending=True, stable=True).indices[:, :k]
+    assert torch.equal(got, order.sort(dim=1).values.int())
+
+
 @pytest.mark.parametrize("batch,tokens,k", [(33, 33000, 700), (33, 4200, 64), (17, 9000, 1100), (4, 12288, 1500),
                                             (4, 12289, 6000), (1, 8192, 1025)])
 def test_decode_topk_by_rows_and_k(batch, tokens, k):
