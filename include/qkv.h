@@ -788,7 +788,9 @@ int qkv_block_scan_scores(const void* query, const void* key_dim_major, const in
 /* The same on the n_scan best of the row's ceil(history / block) block scores
  * (f32 [rows, bscore_ld], the selection of qkv_topk: lowest index first on
  * ties, ascending), selected in the launch and written to blocks; at most
- * 1024 blocks. */
+ * 1024 blocks.  qkv_block_scan_selects: 1 where this one launch is faster than
+ * qkv_topk_ws and qkv_block_scan_scores (the results are the same). */
+int qkv_block_scan_selects(int64_t rows, int64_t history, int64_t block, int64_t n_scan);
 int qkv_block_select_scan_scores(const void* query, const void* key_dim_major, const int64_t* kdm_strides,
                                  const void* key, const int64_t* k_strides, int64_t batch, int64_t q_heads,
                                  int64_t kv_heads, int64_t history, int64_t head_dim, const float* bscore,

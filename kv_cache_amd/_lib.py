@@ -112,6 +112,7 @@ _PROTOTYPES = {
                                 _vp, _i64, _i32, _vp]),
     "qkv_block_scan_scores": (_i32, [_vp, _vp, _P(_i64), _vp, _P(_i64), _i64, _i64, _i64, _i64, _i64, _vp, _i64,
                                      _i64, _i64, _f32, _vp, _vp, _i64, _i32, _vp]),
+    "qkv_block_scan_selects": (_i32, [_i64, _i64, _i64, _i64]),
     "qkv_block_select_scan_scores": (_i32, [_vp, _vp, _P(_i64), _vp, _P(_i64), _i64, _i64, _i64, _i64, _i64, _vp,
                                             _i64, _vp, _i64, _i64, _i64, _f32, _vp, _vp, _i64, _i32, _vp]),
     "qkv_block_max_partial_scores": (_i32, [_vp, _vp, _P(_i64), _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp,

@@ -32,7 +32,6 @@ from .int4 import block_topk, topk_workspace
 from .reuse import dim_major_append, token_attention
 
 QBB, BREP = 0, 1   # QKV_BLOCK_QBB, QKV_BLOCK_BREP
-SCAN_SELECT_BLOCKS = 1024   # rows of at most this many blocks select inside the scan's launch
 QBORACLE = 2       # block maxima of the partial scores: no per-block metadata
 
 
@@ -219,7 +218,7 @@ class BlockSelectDecodeStep:
             # scan computes for every scanned token; the general one (ws_need > 0)
             # computes them for its candidates only
             full = self.full[: self.rows * n_tok] if ws_need == 0 else None
-            if nb <= SCAN_SELECT_BLOCKS:   # the scan's launch selects its blocks
+            if lib.qkv_block_scan_selects(self.rows, history, self.block, n_scan):   # in the scan's launch
                 _lib.check(lib.qkv_block_select_scan_scores(
                     q.data_ptr(), self.kdm.data_ptr(), _lib.strides(*self.kdm.stride()), key.data_ptr(), ks,
                     self.batch, self.q_heads, self.kv_heads, history, self.head_dim, self.bscore.data_ptr(),

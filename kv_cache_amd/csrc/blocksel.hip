@@ -296,12 +296,13 @@ __global__ __launch_bounds__(kBT) void block_scores_kernel(
 // SELV > 0: the blocks are not given; every workgroup of a row selects the
 // n_scan best of the row's nb block scores into LDS (the selection of
 // qkv_topk, SELV keys per thread, repeated by the row's few workgroups instead
-// of launched) and the first writes them to `blocks`.  The token's whole K row
-// (for `full`) and its values on the selected dims are all in flight before
-// either is summed.  32 rows, 513 blocks of 64, 16 scanned, with the
-// selection: 10.9 us (4.2 + 9.0 us as two launches with the row loads behind
-// the partial score).
-template <bool F16, int SELV>
+// of launched) and the first writes them to `blocks`.  AHEAD: the token's whole
+// K row (for `full`) and its values on the selected dims are all in flight
+// before either is summed; the row is held in 64 registers meanwhile, so that
+// fewer workgroups run at once.  32 rows, 513 blocks of 64, 16 scanned, with
+// the selection: 10.9 us (4.2 + 9.0 us as two launches with the row loads
+// behind the partial score).
+template <bool F16, int SELV, bool AHEAD>
 __global__ __launch_bounds__(kBT) void scan_partial_kernel(
     const uint16_t* __restrict__ query, const uint16_t* __restrict__ kdm, int q_heads, int group, int64_t db,
     int64_t dh, int64_t dd, int32_t* __restrict__ blocks, int n_scan, int block, int history, int count,
@@ -328,8 +329,9 @@ __global__ __launch_bounds__(kBT) void scan_partial_kernel(
   const bool in = tok >= 0 && tok < history;
   // (positions without a token load the first one's row, unused)
   uint4 x[kHD / 8];
-  if (full) {   // uniform
-    const uint4* kr = reinterpret_cast<const uint4*>(key + b * sb + (h / group) * sh + static_cast<int64_t>(in ? tok : 0) * st);
+  const uint16_t* krow = key + b * sb + (h / group) * sh + static_cast<int64_t>(in ? tok : 0) * st;
+  if (AHEAD && full) {   // uniform
+    const uint4* kr = reinterpret_cast<const uint4*>(krow);
 #pragma unroll
     for (int c = 0; c < kHD / 8; ++c) x[c] = kr[c];
   }
@@ -350,8 +352,11 @@ __global__ __launch_bounds__(kBT) void scan_partial_kernel(
     }
   }
   out[static_cast<int64_t>(row) * out_ld + p] = acc;
-  if (full)   // the full-D score the rerank ranks its candidates by (every scanned position)
-    full[static_cast<int64_t>(row) * out_ld + p] = in ? full_sum<F16>(x, q_s, scaling) : -__builtin_huge_valf();
+  if (full) {   // the full-D score the rerank ranks its candidates by (every scanned position)
+    float f = -__builtin_huge_valf();
+    if (in) f = AHEAD ? full_sum<F16>(x, q_s, scaling) : full_score<F16>(krow, q_s, scaling);
+    full[static_cast<int64_t>(row) * out_ld + p] = f;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -865,11 +870,23 @@ QKV_EXPORT int qkv_block_scores(int kind, const void* query, const void* key, co
 #undef QKV_BLOCK_SCORES
 }
 
-// Block scores of at most this many blocks select inside the scan's launch:
-// 32 rows x 513 blocks, 4 workgroups a row, 39.7 -> 38.7 us a layer; 256 rows
-// x 250, 2 a row, 48.4 -> 45.9; past it a row has more workgroups to repeat a
-// longer selection (96 rows x 2063, 16 a row, 88.8 -> 90.2).
+// The longest row of block scores the scan's launch selects from.
 constexpr int64_t kScanSelectBlocks = kBT * 4;
+
+// Whether the scan's launch should select its blocks: its workgroups all run
+// at once (4 of 256 threads a CU), so that the selections they repeat cost one
+// selection's time.  us of one launch and of two: 32 rows x 32 workgroups, 500
+// blocks of 64, 18.5 and 20.0, x 40 25.2 and 21.9; 256 rows x 4 19.0 and 20.6, x 6
+// 28.3 and 27.0 (250 blocks 36.0 and 31.4).  From 1024 rows the launch of its own
+// takes one wave per row: 125 blocks 20.2 and 20.6, 250 23.1 and 20.6, 500 19.2
+// and 21.6.
+constexpr int64_t kScanAtOnce = 1024;
+QKV_EXPORT int qkv_block_scan_selects(int64_t rows, int64_t history, int64_t block, int64_t n_scan) {
+  if (rows <= 0 || history <= 0 || block <= 0 || n_scan <= 0) return 0;
+  const int64_t nb = cdiv(history, block);
+  if (rows >= 1024 && nb > 128 && nb <= 256) return 0;
+  return nb <= kScanSelectBlocks && rows * cdiv(n_scan * block, kBT) <= kScanAtOnce ? 1 : 0;
+}
 
 // qkv_block_scan_scores, or with bscore its selecting form.
 static int run_scan(const char* what, const void* query, const void* key_dim_major, const int64_t* kdm_strides,
@@ -890,8 +907,8 @@ static int run_scan(const char* what, const void* query, const void* key_dim_maj
     return fail(QKV_ERR_INVALID, "%s: K rows must be contiguous and 16-byte aligned", what);
   const int count = static_cast<int>(std::min<int64_t>(std::max<int64_t>(dim_count, 1), kHD));
   dim3 grid(static_cast<unsigned>(cdiv(n_scan * block, kBT)), static_cast<unsigned>(batch * q_heads));
-  auto launch = [&](auto ff, auto vv) {
-    scan_partial_kernel<decltype(ff)::value, decltype(vv)::value><<<grid, kBT, 0, static_cast<hipStream_t>(stream)>>>(
+  auto launch = [&](auto ff, auto vv, auto ahead) {
+    scan_partial_kernel<decltype(ff)::value, decltype(vv)::value, decltype(ahead)::value><<<grid, kBT, 0, static_cast<hipStream_t>(stream)>>>(
         static_cast<const uint16_t*>(query), static_cast<const uint16_t*>(key_dim_major), static_cast<int>(q_heads),
         static_cast<int>(q_heads / kv_heads), kdm_strides[0], kdm_strides[1], kdm_strides[2], blocks,
         static_cast<int>(n_scan), static_cast<int>(block), static_cast<int>(history), count, out, out_ld,
@@ -900,8 +917,11 @@ static int run_scan(const char* what, const void* query, const void* key_dim_maj
     return check_launch(what);
   };
   return with_half(f16, [&](auto ff) {
-    if (!bscore) return launch(ff, std::integral_constant<int, 0>{});
-    return launch(ff, std::integral_constant<int, 4>{});
+    if (bscore) return launch(ff, std::integral_constant<int, 4>{}, std::true_type{});
+    // the row loads ahead while they fit beside few workgroups: with the selection's
+    // launch, 64 rows x 8 workgroups 14.4 us (14.9 behind the partial score), x 24 27.3 (26.1)
+    const std::integral_constant<int, 0> given{};
+    return grid.x * grid.y <= kScanAtOnce / 2 ? launch(ff, given, std::true_type{}) : launch(ff, given, std::false_type{});
   });
 }
 

@@ -181,3 +181,12 @@ def test_reuse_block_final_count():
     assert lib.qkv_reuse_final_count(37, 50, 0, 0.1, 0) == 4 + 37
     assert lib.qkv_reuse_block_final_count(0, 16, 0, 0, 0.1, 1) == -1
     assert lib.qkv_reuse_block_final_count(10, 0, 0, 0, 0.1, 1) == -1
+
+
+@pytest.mark.parametrize("rows,nb,block,n_scan,selects", [
+    (32, 513, 64, 16, 1), (32, 500, 64, 128, 1), (32, 500, 64, 129, 0), (256, 1000, 16, 64, 1), (256, 1000, 16, 65, 0),
+    (1, 1024, 16, 100, 1), (1, 1025, 16, 100, 0), (1024, 128, 16, 16, 1), (1024, 129, 16, 16, 0),
+    (1024, 256, 16, 16, 0), (1024, 257, 16, 16, 1), (1025, 257, 16, 16, 0)])
+def test_scan_selects_while_its_workgroups_run_at_once(rows, nb, block, n_scan, selects):
+    assert lib.qkv_block_scan_selects(rows, nb * block, block, n_scan) == selects
+    assert lib.qkv_block_scan_selects(rows, nb * block - block + 1, block, n_scan) == selects

@@ -286,11 +286,13 @@ def test_rerank_with_and_without_scan_full_scores(mode, t):
         assert torch.equal(ids, want_ids), full is None
 
 
-@pytest.mark.parametrize("nb,n_scan,block", [(1, 1, 16), (256, 7, 4), (257, 257, 4), (1000, 90, 16), (1024, 16, 2)])
+# (batch 2: few workgroups; batch 9 with 70 x 64 tokens scanned: 648, past those whose rows are loaded ahead)
+@pytest.mark.parametrize("nb,n_scan,block,b", [(1, 1, 16, 2), (256, 7, 4, 2), (257, 257, 4, 2), (1000, 90, 16, 2),
+                                               (1024, 16, 2, 2), (90, 70, 64, 9), (90, 56, 64, 9)])
 @pytest.mark.parametrize("full", [True, False])
-def test_scan_that_selects_equals_topk_then_scan(nb, n_scan, block, full):
+def test_scan_that_selects_equals_topk_then_scan(nb, n_scan, block, b, full):
     lib = _lib.load()
-    b, hkv, hq, t = 2, 2, 4, nb * block - min(block - 1, 1)
+    hkv, hq, t = 2, 4, nb * block - min(block - 1, 1)
     k, _, g = _kv(b, hkv, t, nb)
     q = torch.randn((b, hq, 128), generator=g).to(torch.bfloat16).to(DEV)
     kd = k.to(DEV)
@@ -314,3 +316,21 @@ def test_scan_that_selects_equals_topk_then_scan(nb, n_scan, block, full):
     for x, y in zip(*outs):
         assert torch.equal(x, y)
     assert lib.qkv_block_select_scan_scores(*head, score.data_ptr(), nb + 3, blocks.data_ptr(), nb + 1, *tail[1:]) == -1
+
+
+@pytest.mark.parametrize("b,t", [(1, 3000), (32, 3000), (64, 700)])   # one launch; too many workgroups; rows
+def test_step_by_launches_of_the_scan(b, t):
+    mode, hq, hkv = "qbb16q8s12cand4", 32, 8
+    k, v, g = _kv(b, hkv, t, b + t)
+    q = torch.randn((b, hq, 128), generator=g).to(torch.bfloat16).to(DEV)
+    step = BS.BlockSelectDecodeStep(mode, b, hq, hkv, 128, t, top_fraction=0.02, protect_sink=2, protect_recent=4)
+    nb, n_scan, _, _ = BS.step_counts(t - 1, step.block, step.scan, step.cand, step.top_fraction)
+    assert bool(_lib.load().qkv_block_scan_selects(b * hq, t - 1, step.block, n_scan)) == (b == 1)
+    out = step(q, k.to(DEV), v.to(DEV), 0.088)
+    mask = step.final_mask()
+    one = BS.BlockSelectDecodeStep(mode, 1, hq, hkv, 128, t, top_fraction=0.02, protect_sink=2, protect_recent=4)
+    for i in (0, b // 2, b - 1):   # each sequence as a step of its own gives it
+        got = one(q[i : i + 1], k[i : i + 1].to(DEV), v[i : i + 1].to(DEV), 0.088)
+        assert torch.equal(one.final_mask()[0], mask[i])
+        assert torch.equal(got[0], out[i])
+        one.reset()
