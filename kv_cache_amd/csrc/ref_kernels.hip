@@ -226,7 +226,15 @@ template <int DT> struct RunPartial {
   static int run(const void* q, const void* k, float* out, int64_t B, int64_t H, int64_t T,
                  int64_t D, const int64_t* ks, int count, hipStream_t st) {
     using E = typename Elem<DT>::T;
-    if (D == 128 && ks[3] == 1) {
+    // A K that no cache holds and few dims: the lines of a row that hold none
+    // of them are not worth reading.  us by rows and by dims, fp32 (4 lines a
+    // row), 32 heads: 2000 tokens, 1 dim, 7.6 and 9.0; 4000, 4 and 5 dims, 13.9 and
+    // 13.4, 16.0; 65536, 5 and 6 dims, 176 and 163, 191.  bf16 (2 lines): 65536,
+    // 1 and 2 dims, 93 and 80, 109; 4 x 8190, 1 dim, 40.1 and 42.7.
+    const int64_t bytes = B * H * T * D * static_cast<int64_t>(sizeof(E));
+    constexpr int64_t kMB = 1 << 20;
+    const int few = DT == QKV_DTYPE_FP32 ? (bytes > 192 * kMB ? 5 : bytes > 48 * kMB ? 4 : 0) : bytes > 384 * kMB ? 1 : 0;
+    if (D == 128 && ks[3] == 1 && count > few) {
       constexpr int tok = kRowWaves * (DT == QKV_DTYPE_FP32 ? 32 : 64);
       dim3 rgrid(static_cast<unsigned>(cdiv(T, tok)), static_cast<unsigned>(B * H));
       partial_scores_rows_kernel<DT><<<rgrid, 64 * kRowWaves, 0, st>>>(

@@ -34,6 +34,20 @@ def test_scores_at_tile_edges(dtype, keys, pad):
         assert np.array_equal(got, want)
 
 
+# both sides of the lines between whole rows and single dims: 61 and 203 MB of fp32, 406 MB of bf16
+@pytest.mark.parametrize("dtype,keys,dims", [(torch.float32, 3900, 4), (torch.float32, 3900, 5), (torch.float32, 13000, 5),
+                                             (torch.float32, 13000, 6), (torch.bfloat16, 52000, 1),
+                                             (torch.bfloat16, 52000, 2)])
+def test_few_dims_of_a_large_history(dtype, keys, dims):
+    g = torch.Generator(device=DEV).manual_seed(keys + dims)
+    k = torch.randn((1, 32, keys, 128), generator=g, device=DEV).to(dtype)
+    q = torch.randn((1, 32, 128), generator=g, device=DEV).to(dtype)
+    got = Q.partial_scores(q, k, dims)
+    for h in (0, 17, 31):
+        want = R.partial_scores(q[:, h : h + 1].float().cpu().numpy(), k[:, h : h + 1].float().cpu().numpy(), dims)
+        assert np.array_equal(got[:, h : h + 1].cpu().numpy(), want)
+
+
 def test_token_ids():
     idx = torch.tensor([0, 5, 6, -1, 2 ** 40, -2 ** 40, 3, 2 ** 32 + 1], device=DEV)
     valid = torch.tensor([1, 1, 1, 1, 1, 1, 0, 1], dtype=torch.uint8, device=DEV)
