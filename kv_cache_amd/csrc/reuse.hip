@@ -108,15 +108,21 @@ __global__ __launch_bounds__(kPartNT) void reuse_partial_kernel(
   }
   const int t0 = (blockIdx.x * kPartNT + tid) * 8;
   if (!HIST && t0 >= history) return;
-  const int nt = max(min(8, history - t0), 0);   // this thread's tokens
-  const E* base = kdm + b * sb + (h / group) * sh + min(t0, history - 1);
-  float* o = out + static_cast<int64_t>(row) * out_ld + t0;
+  // This thread's tokens are the last `8 - skip` of the eight from ts on: the
+  // row's last n < 8 tokens are loaded with the 8 - n before them, which is as
+  // fast as any eight, where element loads at clamped addresses were on the
+  // launch's critical path (32 rows x 32767 tokens, S = 8 7.1 us, 5.7 now; S = 64
+  // 32.0 and 18.9).
+  const int ts = max(min(t0, history - 8), 0);
+  const int skip = t0 < history ? t0 - ts : 8;
+  const E* base = kdm + b * sb + (h / group) * sh + ts;
+  float* o = out + static_cast<int64_t>(row) * out_ld + ts;
   float acc[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
-  if (nt == 0) {
+  if (skip == 8) {
     // (HIST: a thread past the row still takes part in the barriers below)
-  } else if (nt == 8) {
+  } else if (history >= 8) {
     // eight dims' loads in flight at once (clamped, in bounds), then the
     // products added in selection order
     for (int s0 = 0; s0 < count; s0 += 8) {
@@ -132,39 +138,29 @@ __global__ __launch_bounds__(kPartNT) void reuse_partial_kernel(
         }
       }
     }
+    if (skip == 0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = acc[i];
-  } else {
-    // the row's last n < 8 tokens: the same order,
-    // every load in flight at once at clamped in-row addresses, then only
-    // the n tokens stored (a load-then-add loop over runtime n waits for
-    // each load in turn)
-    const int n = min(8, history - t0);
-    for (int s0 = 0; s0 < count; s0 += 8) {
-      float v[8][8];
+      for (int i = 0; i < 8; ++i) o[i] = acc[i];
+    } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const E* p = base + sel_idx[min(s0 + j, count - 1)] * sd;
+      for (int i = 0; i < 8; ++i)
+        if (i >= skip) o[i] = acc[i];
+    }
+  } else {   // a row of fewer than eight tokens: in order, one element at a time
+    for (int s = 0; s < count; ++s) {
+      const E* p = base + sel_idx[s] * sd;
+      const float qs = sel_q[s];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[j][i] = Elem<DT>::load(p + min(i, n - 1));
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (s0 + j < count) {
-          const float qs = sel_q[s0 + j];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc[i] = acc[i] + qs * v[j][i];
-        }
-      }
+      for (int i = 0; i < 8; ++i) acc[i] = acc[i] + qs * Elem<DT>::load(p + min(i, history - 1));
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      if (i < n) o[i] = acc[i];
+      if (i < history) o[i] = acc[i];
   }
   if constexpr (HIST) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      if (i < nt) atomicAdd(&hist_s[f32_sortable(acc[i]) >> (32 - kCandBits)], 1);
+      if (i >= skip && ts + i < history) atomicAdd(&hist_s[f32_sortable(acc[i]) >> (32 - kCandBits)], 1);
     __syncthreads();
     int* hrow = hist + static_cast<int64_t>(row) * kCandBins;
 #pragma unroll
@@ -1954,8 +1950,13 @@ template <int DT> struct RunReusePartial {
                  const uint8_t* gate = nullptr, int gate_refresh = 0, int* hist = nullptr) {
     using E = typename Elem<DT>::T;
     dim3 grid(static_cast<unsigned>(cdiv(T, 8 * kPartNT)), static_cast<unsigned>(B * Hq));
+    // With many dims the heads of a KV head share most of what they read: four
+    // workgroups a CU (by LDS that nothing uses) keep it in the caches until all
+    // have.  32 rows x 131072 tokens, S = 128: 126 us, 131 without, S = 8 17.3 and
+    // 16.6; 96 x 32000, S = 64 50.4 and 52.0, S = 16 19.3 and 18.6.
+    const size_t lds = count > 16 ? 32000 - (hist ? sizeof(int) * kCandBins : 0) : 0;
 #define QKV_REUSE_PARTIAL(HH)                                                                                  \
-  reuse_partial_kernel<DT, HH><<<grid, kPartNT, 0, st>>>(static_cast<const E*>(q), static_cast<const E*>(kdm),     \
+  reuse_partial_kernel<DT, HH><<<grid, kPartNT, lds, st>>>(static_cast<const E*>(q), static_cast<const E*>(kdm),     \
                                                      static_cast<int>(Hq), static_cast<int>(Hq / Hkv),         \
                                                      static_cast<int>(T), static_cast<int>(D), count, ks[0],   \
                                                      ks[1], ks[2], out, out_ld, gate, gate_refresh,            \

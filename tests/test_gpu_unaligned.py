@@ -24,7 +24,8 @@ def copy_at(k, offset, pad):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("offset,pad", [(0, 0), (1, 1), (3, 4), (7, 8)])
-@pytest.mark.parametrize("batch,hist", [(1, 7), (1, 2049), (32, 1003)])   # (32 x 4 rows: the one-launch candidates)
+@pytest.mark.parametrize("batch,hist", [(1, 1), (1, 7), (1, 8), (1, 9), (1, 2049), (1, 2055),
+                                        (32, 1003)])   # (32 x 4 rows: the one-launch candidates)
 def test_partial_scores_at_any_alignment(dtype, offset, pad, batch, hist):
     g = torch.Generator().manual_seed(hist + offset)
     hq, hkv, d, dims = 4, 2, 128, 12
