@@ -194,9 +194,29 @@ def test_topk_matches_oracle(n, k):
     assert np.array_equal(got, O.topk_lowest_index(vals.numpy(), k))
 
 
+def chunk_list_topk(vals, k, out=None, ws=None):
+    """block_topk with a workspace of the chunk lists' size (at most 64 chunks, chunks * k <= 32768), which
+    holds no row histogram: the one-launch form where rows * chunks <= 256, else three launches."""
+    from kv_cache_amd import _lib
+    lib = _lib.load()
+    rows, n = vals.shape
+    chunks = -(-n // 4096)
+    assert chunks <= 64 and chunks * k <= 32768
+    need = rows * chunks * (66 + 2 * k + 1) * 4
+    assert need < lib.qkv_topk_workspace_bytes(rows, n, k)
+    if ws is None:
+        ws = torch.empty(need // 4, device=DEV)
+    if out is None:
+        out = torch.empty((rows, k), dtype=torch.int32, device=DEV)
+    assert ws.numel() * 4 >= need
+    _lib.check(lib.qkv_topk_ws(vals.data_ptr(), rows, n, vals.stride(0), k, out.data_ptr(), ws.data_ptr(), need,
+                               _lib.stream_of(vals)))
+    return out
+
+
 def test_topk_staged_equals_single_workgroup():
-    # Rows longer than 4096 keys go through the staged reduction; qkv_topk
-    # (one workgroup per row) must give the same indices.
+    # Rows longer than 4096 keys go through the row histogram or the chunk
+    # lists; qkv_topk (one workgroup per row) must give the same indices.
     from kv_cache_amd import _lib
     lib = _lib.load()
     g = torch.Generator().manual_seed(77)
@@ -206,8 +226,8 @@ def test_topk_staged_equals_single_workgroup():
         want = torch.empty((5, k), dtype=torch.int32, device=DEV)
         _lib.check(lib.qkv_topk(vals.data_ptr(), 5, 70000, 70000, k, want.data_ptr(), _lib.stream_of(vals)))
         assert lib.qkv_topk_workspace_bytes(5, 70000, k) > 0
-        got = K.block_topk(vals, k)
-        assert torch.equal(got, want)
+        assert torch.equal(K.block_topk(vals, k), want)
+        assert torch.equal(chunk_list_topk(vals, k), want)
 
 
 def _adversarial_rows(n, seed):
@@ -243,8 +263,9 @@ def test_topk_long_rows_adversarial(n, k):
     # pass more than k keys per chunk, one-lane rows leave most chunks empty,
     # a partial last chunk adds no bound
     vals = _adversarial_rows(n, n + k)
-    got = K.block_topk(vals.to(DEV), k).cpu().numpy()
-    assert np.array_equal(got, O.topk_lowest_index(vals.numpy(), k))
+    want = O.topk_lowest_index(vals.numpy(), k)
+    assert np.array_equal(K.block_topk(vals.to(DEV), k).cpu().numpy(), want)
+    assert np.array_equal(chunk_list_topk(vals.to(DEV), k).cpu().numpy(), want)
 
 
 def test_topk_long_rows_one_chunk_over_k():
@@ -255,8 +276,9 @@ def test_topk_long_rows_one_chunk_over_k():
     vals[0, 8192:12288] += 10.0                 # chunk 2: 4096 keys above every other chunk's
     vals[1, 5::4096] = 100.0                   # one huge key per chunk
     vals[2, 4096 * 15:] = -float("inf")        # the last chunk -inf only
-    got = K.block_topk(vals.to(DEV), k).cpu().numpy()
-    assert np.array_equal(got, O.topk_lowest_index(vals.numpy(), k))
+    want = O.topk_lowest_index(vals.numpy(), k)
+    assert np.array_equal(K.block_topk(vals.to(DEV), k).cpu().numpy(), want)
+    assert np.array_equal(chunk_list_topk(vals.to(DEV), k).cpu().numpy(), want)
 
 
 def test_topk_long_rows_three_launch_grid():
@@ -264,7 +286,7 @@ def test_topk_long_rows_three_launch_grid():
     # launches (the one-launch form needs every workgroup resident)
     n, k = 131072, 1024
     vals = torch.cat([_adversarial_rows(n, 11), _adversarial_rows(n, 12)[:2]])   # 9 rows x 32 chunks
-    got = K.block_topk(vals.to(DEV), k).cpu().numpy()
+    got = chunk_list_topk(vals.to(DEV), k).cpu().numpy()
     assert np.array_equal(got, O.topk_lowest_index(vals.numpy(), k))
 
 
@@ -277,7 +299,7 @@ def test_topk_one_launch_workspace_reuse():
                        (8, 131072, 1)]:
         vals = torch.randn((rows, n), generator=g)
         vals[rows // 2, ::2] = 7.0   # ties across every chunk
-        got = K.block_topk(vals.to(DEV), k, workspace=ws).cpu().numpy()
+        got = chunk_list_topk(vals.to(DEV), k, ws=ws).cpu().numpy()
         assert np.array_equal(got, O.topk_lowest_index(vals.numpy(), k)), (rows, n, k)
 
 
@@ -292,7 +314,7 @@ def test_topk_one_launch_ticket_pool_wraps():
     out = torch.empty((2, 64), dtype=torch.int32, device=DEV)
     ws = K.topk_workspace(2, 9000, 64, DEV)
     for i in range(4200):
-        K.block_topk(dev[i % 3], 64, out=out, workspace=ws)
+        chunk_list_topk(dev[i % 3], 64, out=out, ws=ws)
         if i % 700 == 0 or i >= 4197:
             assert np.array_equal(out.cpu().numpy(), want[i % 3]), i
 
@@ -308,12 +330,12 @@ def test_topk_one_launch_graph_replays():
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(s):
-        K.block_topk(x.normal_(), k, out=out, workspace=ws)
+        chunk_list_topk(x.normal_(), k, out=out, ws=ws)
     torch.cuda.current_stream().wait_stream(s)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        K.block_topk(x, k, out=out, workspace=ws)
+        chunk_list_topk(x, k, out=out, ws=ws)
     for rep in range(4):
         host = torch.randn((rows, n), generator=g)
         if rep == 2:
@@ -336,13 +358,13 @@ def test_topk_one_launch_wait_limit_zero():
     vals = _adversarial_rows(n, 41)
     _lib.check(lib.qkv_topk_set_wait_limit(0))
     try:
-        got = K.block_topk(vals.to(DEV), k).cpu().numpy()
-        got2 = K.block_topk(vals.to(DEV), 3).cpu().numpy()
+        got = chunk_list_topk(vals.to(DEV), k).cpu().numpy()
+        got2 = chunk_list_topk(vals.to(DEV), 3).cpu().numpy()
     finally:
         _lib.check(lib.qkv_topk_set_wait_limit(-1))
     assert np.array_equal(got, O.topk_lowest_index(vals.numpy(), k))
     assert np.array_equal(got2, O.topk_lowest_index(vals.numpy(), 3))
-    got = K.block_topk(vals.to(DEV), k).cpu().numpy()   # default wait again
+    got = chunk_list_topk(vals.to(DEV), k).cpu().numpy()   # default wait again
     assert np.array_equal(got, O.topk_lowest_index(vals.numpy(), k))
 
 
