@@ -1208,7 +1208,6 @@ constexpr int64_t kBigMax = 192 * 1024;    // positions whose bitset fits beside
 constexpr int kBigSlices = 64;             // slices per row, one lane of a wave each
 constexpr int kBigState = kBigSlices + 8;  // ints per row: the slices' counts, then the ticket
 constexpr int kBigStride = kHistBins + kBigState;   // ints per row of histogram and state
-constexpr int kBigListed = 8 * 1024;       // keys of the boundary bin resolved in registers
 
 __global__ __launch_bounds__(256) void topk_clear_kernel(int4* __restrict__ p, int64_t n) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -1493,20 +1492,20 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
   // The bin holds at least `rank` keys; a histogram that was not zero when the
   // row was counted may say otherwise, and then none is taken.
   const bool over = over_sh;
-  if (__builtin_expect(over || m > kBigListed || m < rank, 0)) {   // uniform
-    if (over || m >= rank)
-      bin_taken_stream(&sh, over ? n : m, rank, bin, n, fw, [&](int p, float& x, int& pos) {
-        if (over) {
-          x = vrow[p];
-          pos = p;
-        } else {
-          from_list(p, x, pos);
-        }
-      });
-  } else if (m <= 1024) bin_taken<1>(&sh, m, rank, bin, n, fw, from_list);
-  else if (m <= 2 * 1024) bin_taken<2>(&sh, m, rank, bin, n, fw, from_list);
-  else if (m <= 4 * 1024) bin_taken<4>(&sh, m, rank, bin, n, fw, from_list);
-  else bin_taken<8>(&sh, m, rank, bin, n, fw, from_list);
+  const bool listed = !over && m >= rank;
+  if (listed && m <= 1024) bin_taken<1>(&sh, m, rank, bin, n, fw, from_list);   // (uniform)
+  else if (listed && m <= 2 * 1024) bin_taken<2>(&sh, m, rank, bin, n, fw, from_list);
+  else if (listed && m <= 4 * 1024) bin_taken<4>(&sh, m, rank, bin, n, fw, from_list);
+  else if (listed && m <= 8 * 1024) bin_taken<8>(&sh, m, rank, bin, n, fw, from_list);
+  else if (listed || over)
+    bin_taken_stream(&sh, over ? n : m, rank, bin, n, fw, [&](int p, float& x, int& pos) {
+      if (over) {
+        x = vrow[p];
+        pos = p;
+      } else {
+        from_list(p, x, pos);
+      }
+    });
   __syncthreads();
   // the taken positions, ascending: consecutive words per thread
   const int wpt = (n_words + 1023) / 1024;
@@ -1518,14 +1517,12 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
   const int incl = wave_incl_scan_dpp(cnt);
   if (lane == 63) wave_cnt[wave] = incl;
   __syncthreads();
-  int p = incl - cnt, taken = 0;
+  int p = incl - cnt;
 #pragma unroll
   for (int w = 0; w < 16; ++w) {
     p += w < wave ? wave_cnt[w] : 0;
-    taken += wave_cnt[w];
   }
   int32_t* orow = out + static_cast<int64_t>(row) * k;
-  for (int at = taken + tid; at < k; at += 1024) orow[at] = -1;   // (not reached from a zero histogram)
   for (int j = 0; j < wpt; ++j) {
     const int w = tid * wpt + j;
     if (w >= n_words) break;
@@ -1534,6 +1531,8 @@ __global__ __launch_bounds__(1024) void topk_slices_kernel(const float* __restri
       ++p;
     }
   }
+  if (tid == 1023)   // the row's end (k, from a histogram that was zero)
+    for (; p < k; ++p) orow[p] = -1;
 }
 
 // Candidates left after a stage over n keys: k from every full chunk, and
