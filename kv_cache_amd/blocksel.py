@@ -135,6 +135,7 @@ class BlockSelectDecodeStep:
         need = lib.qkv_sparse_attention_workspace_bytes(batch, q_heads, q_heads, head_dim, self.n_out_max, 1)
         self.attn_ws = torch.zeros((need + 3) // 4, dtype=torch.float32, device=device)
         self.out = torch.empty((batch, q_heads, head_dim), dtype=dtype, device=device)
+        self.scan_sizes, self.scan_selects = None, 0   # the sizes qkv_block_scan_selects was asked for, its answer
         self.reset()
 
     def reset(self) -> None:
@@ -218,7 +219,10 @@ class BlockSelectDecodeStep:
             # scan computes for every scanned token; the general one (ws_need > 0)
             # computes them for its candidates only
             full = self.full[: self.rows * n_tok] if ws_need == 0 else None
-            if lib.qkv_block_scan_selects(self.rows, history, self.block, n_scan):   # in the scan's launch
+            if self.scan_sizes != (nb, n_scan):   # (asked once per size, not per token)
+                self.scan_sizes = (nb, n_scan)
+                self.scan_selects = lib.qkv_block_scan_selects(self.rows, history, self.block, n_scan)
+            if self.scan_selects:   # the scan's launch selects its blocks
                 _lib.check(lib.qkv_block_select_scan_scores(
                     q.data_ptr(), self.kdm.data_ptr(), _lib.strides(*self.kdm.stride()), key.data_ptr(), ks,
                     self.batch, self.q_heads, self.kv_heads, history, self.head_dim, self.bscore.data_ptr(),
