@@ -207,7 +207,8 @@ int qkv_topk(const float* values, int64_t rows, int64_t n, int64_t ld, int64_t k
  * for the longest row serves them all (the size functions below that are
  * built on it hold to the same for a shorter history).  0 for n <= 4096; for
  * n <= 196608 a 4096-bin histogram, a bitset and the slices' lists per row,
- * whatever k; past that no less than this for 196608 and what the chunk lists
+ * whatever k (from 512 rows also what the chunk lists below take, where n is
+ * past 32 chunks); past that no less than this for 196608 and what the chunk lists
  * below take: for rows of at most 64 chunks of 4096 keys with ceil(n/4096) * k
  * <= 32768, per chunk a 66-word histogram window and a list of k (value,
  * index) pairs with its count, else two candidate buffers of rows * (k *
@@ -219,11 +220,12 @@ int64_t qkv_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k);
 
 /* qkv_topk with a caller-owned workspace (16-byte aligned, contents
  * irrelevant; calls sharing a workspace must not overlap in time).  Rows of
- * 4097 to 196608 keys, any k: three launches clear a histogram per row, count
- * the keys' top 12 bits into it, and select from slices of the row.  With
- * k <= 1024, longer rows, and calls with a workspace smaller than the row
- * histogram's but enough for the chunk lists, are split into
- * 4096-key chunks; with k > 1024 such calls take qkv_topk.  Rows
+ * 4097 to 196608 keys (with k > 1024: 12289 to 196608): three launches clear
+ * a histogram per row, count the keys' top 12 bits into it, and select from
+ * slices of the row.  With k <= 1024, longer rows, 512 and more rows with
+ * more than 64 chunks or chunks * k > 32768, and calls with a workspace
+ * smaller than the row histogram's but enough for the chunk lists, are split
+ * into 4096-key chunks; with k > 1024 all other calls take qkv_topk.  Rows
  * of at most 64 chunks with chunks * k <= 32768: every chunk histograms its
  * keys (1/8-octave bins) around its own k-th key, the row's floor is the bin
  * where the merged count from the top reaches k, each chunk keeps its keys

@@ -300,7 +300,7 @@ __global__ __launch_bounds__(kBT) void block_scores_kernel(
 // K row (for `full`) and its values on the selected dims are all in flight
 // before either is summed; the row is held in 64 registers meanwhile, so that
 // fewer workgroups run at once.  32 rows, 513 blocks of 64, 16 scanned, with
-// the selection: 10.9 us (4.2 + 9.0 us as two launches with the row loads
+// the selection: 11.0 us (4.2 + 9.0 us as two launches with the row loads
 // behind the partial score).
 template <bool F16, int SELV, bool AHEAD>
 __global__ __launch_bounds__(kBT) void scan_partial_kernel(

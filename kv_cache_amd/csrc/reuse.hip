@@ -45,7 +45,7 @@ constexpr int kMaskTile = 4096;   // tokens per workgroup in reuse_mask_kernel
 // EV:2018-2042; dims chosen as QK:120-145).  Eight tokens per thread, one
 // 16-byte load per dim at any alignment: a copy whose rows hold an odd
 // number of tokens reads at the same rate (128 rows x 16410 tokens, S = 8:
-// 28.7 us with element loads there, 12.8 us now).
+// 28.7 us with element loads there, 10.8 us now).
 // HIST: each score's top 12 order-preserving bits (the first radix digit of
 // the candidate selection, kCandBins bins) are also counted into
 // hist[row * kCandBins + digit], through a workgroup histogram in LDS and
@@ -1832,9 +1832,9 @@ int with_wide_vpl(int64_t n, F&& f) {
 // The same in finer steps, for kernels that always work on the whole row: a
 // wave owns 64 * VPL consecutive positions, so a row a little longer than a
 // coarse step would leave half the workgroup's waves without keys and give
-// the others twice as many: 128 rows of 16410 scores at 32 values a thread
-// 21.4 us, at 20 18.6; exact candidate attention over 256 rows of 4000 at 16
-// 42.5 us a layer, at 4 38.9.
+// the others twice as many.  Exact candidate attention, us a layer in these
+// steps and in the coarse ones: 128 rows of 16410 scores 44.0 and 47.9, of
+// 8999 32.0 and 33.5, 256 rows of 3999 27.2 and 29.9.
 template <typename F>
 int with_wide_vpl_fine(int64_t n, F&& f) {
   if (n <= 4 * kWideNT) return f(std::integral_constant<int, 4>{});

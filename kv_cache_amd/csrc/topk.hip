@@ -1197,8 +1197,8 @@ __global__ __launch_bounds__(1024) void topk_fused_kernel(const float* __restric
 // irrelevant), a state the caller keeps is put back to zero by the last slice.
 // Bound by latency (the launch, the histogram and keys, the ticket, the last
 // slice's two passes and its output): 11.6 us at 32 rows x 20010 keys with k =
-// 1001 (13.7 in topk_fused_kernel), 12.2 at 8 rows x 131072 with k = 1024
-// (17.4) and at 8 x 131071 with k = 6554 (222 us, one workgroup per row).
+// 1001 (13.7 in topk_fused_kernel), 11.5 at 8 rows x 131072 with k = 1024
+// (17.4) and 12.2 at 8 x 131071 with k = 6554 (222 us, one workgroup per row).
 // Rows with a large share of their keys in one bin (1/8 octave) take longer: 8
 // rows x 131072 keys 100 + 0.5 z, k = 64 and 1000, 31 and 113 us with the two
 // launches before (163 where the last slice reads the row; chunk lists 35 and
@@ -1550,12 +1550,13 @@ bool filtered(int64_t n, int64_t k) {
   return staged(n, k) && chunks <= kFilterMaxChunks && chunks * k <= kFilterMaxLists;
 }
 
-// Rows that take the row histogram and slices: every row longer than the
-// one-workgroup selections take.  Decode steps of a token selection that
-// keeps its state, against the chunk lists (us a layer): 8 rows x 4500 23.6
-// (33.1), 8 x 8000 24.3 (27.0), 64 x 7000 29.9 (32.4), 8 x 131072 32.8
-// (39.3), 256 x 5000 33.0 (33.1); block maxima, which also pay the clearing
-// and the counting launch: 8 rows x 6250 37.1 (45.2), 64 x 8192 73.5 (79.2).
+// Rows that the row histogram and slices can take (topk_takes_row_hist says
+// which of them do): every row longer than the one-workgroup selections take.
+// Whole decode steps of a token selection that keeps its state, and in the
+// tree whose steps took the chunk lists (us a layer): 8 rows x 4500 25.2
+// (34.5), 8 x 8000 24.8 (27.5), 64 x 7000 29.2 (31.6), 8 x 131072 31.4
+// (37.9), 256 x 5000 38.7 (48.7); block maxima, which also pay the clearing
+// and the counting launch: 8 rows x 6250 36.8 (43.5), 64 x 8192 92.5 (97.1).
 // The chunk lists stay for rows past kBigMax and for calls whose workspace
 // was sized for them.
 bool big(int64_t n) { return n > kStageChunk && n <= kBigMax; }
